@@ -103,6 +103,20 @@ int sffft_spectrum(const float* k, int H, int L, const sffft_plan* plan, void* k
  * gradients are, is sffft_conv_* of x with this spectrum: no time reversal of x or z. */
 int sffft_spectrum_conj(const float* k, int H, int L, const sffft_plan* plan, void* kf, void* work, void* stream);
 
+/* Filter gradient of the causal convolution,
+ *   dk[h,j] = sum_b sum_{n>=j} dy[b,h,n] u[b,h,n-j],  j < L,
+ * for L a power of two in [128, 16384] and any B, H. No counterpart in the reference: it serves
+ * the gradient of sffft_conv_* with respect to k. u, dy are [B][H][L] (fp32 or bf16, rows of any
+ * element alignment), dk is [H][L] fp32, 16-byte aligned, and may overlap neither input. The
+ * transforms and sums are fp32 (about 2e-7 rel-L2 against fp64). `work` (16-byte aligned,
+ * clobbered) must hold sffft_filter_grad_work_bytes(B, H, L) bytes and may be NULL if that is 0.
+ * Needs no plan and no table: the first call may be captured. */
+size_t sffft_filter_grad_work_bytes(int B, int H, int L);
+int sffft_filter_grad_f32(const float* u, const float* dy, float* dk, void* work, size_t work_bytes, int B, int H,
+                          int L, void* stream);
+int sffft_filter_grad_bf16(const uint16_t* u, const uint16_t* dy, float* dk, void* work, size_t work_bytes, int B,
+                           int H, int L, void* stream);
+
 /* sffft_spectrum without the `work` argument, for callers that cannot allocate (code under
  * HIP graph capture, serving loops, harnesses that forbid hipMalloc). No counterpart in the
  * reference. It stages the channels through a static device array of 32 MiB per GPU (held

@@ -110,6 +110,9 @@ def load_library(path: str) -> ctypes.CDLL:
         "sffft_spectrum_bytes": (sz, [ci, ci]),
         "sffft_spectrum": (ci, [vp, ci, ci, P, vp, vp, vp]),
         "sffft_spectrum_conj": (ci, [vp, ci, ci, P, vp, vp, vp]),
+        "sffft_filter_grad_work_bytes": (sz, [ci, ci, ci]),
+        "sffft_filter_grad_f32": (ci, [vp, vp, vp, vp, sz, ci, ci, ci, vp]),
+        "sffft_filter_grad_bf16": (ci, [vp, vp, vp, vp, sz, ci, ci, ci, vp]),
         "sffft_spectrum_from_natural": (ci, [vp, ci, ci, P, vp, vp]),
         "sffft_spectrum_from_natural_complex": (ci, [vp, ci, ci, P, vp, vp]),
         "sffft_spectrum_noalloc": (ci, [vp, ci, ci, P, vp, vp]),

@@ -791,6 +791,24 @@ bool span_overlap(const void* a, size_t na, const void* b, size_t nb) {
 }
 bool aligned8(const void* p) { return ((uintptr_t)p & 7u) == 0; }
 
+size_t filter_grad_work(int B, int H, int L) {
+  const int parts = filter_grad_parts(B, H, L);
+  return parts > 1 ? (size_t)parts * H * L * 4 : 0;
+}
+
+int filter_grad_call(const void* u, const void* dy, float* dk, void* work, size_t wbytes, int B, int H, int L, int io,
+                     void* stream) {
+  if (!u || !dy || !dk || B < 1 || H < 1 || (long long)B * H > INT_MAX || filter_grad_parts(B, H, L) < 1)
+    return SFFFT_EINVAL;
+  const size_t need = filter_grad_work(B, H, L), in = (size_t)B * H * L * (io ? 2 : 4), out = (size_t)H * L * 4;
+  if (((uintptr_t)u | (uintptr_t)dy) & (io ? 1u : 3u) || !aligned16(dk)) return SFFFT_EINVAL;
+  if (span_overlap(dk, out, u, in) || span_overlap(dk, out, dy, in)) return SFFFT_EINVAL;
+  if (need && (!work || wbytes < need || !aligned16(work) || span_overlap(work, need, u, in) ||
+               span_overlap(work, need, dy, in) || span_overlap(work, need, dk, out)))
+    return SFFFT_EINVAL;
+  return hip_status(filter_grad(u, dy, dk, work, B, H, L, io, (hipStream_t)stream), "filter gradient launch");
+}
+
 // Validated 1-D transform layout; *extent: extent of x / X in complex elements. Two layout
 // families are supported, both one-to-one (no two (sequence, element) pairs at one
 // address): each sequence whole before the next (dist >= N * stride), or the sequences
@@ -828,6 +846,20 @@ int circconv2d_layout(int B, int H, int N0, int N1, long long* elems, long long*
   return SFFFT_OK;
 }
 }  // namespace
+
+size_t sffft_filter_grad_work_bytes(int B, int H, int L) {
+  return B < 1 || H < 1 ? 0 : filter_grad_work(B, H, L);
+}
+
+int sffft_filter_grad_f32(const float* u, const float* dy, float* dk, void* work, size_t work_bytes, int B, int H,
+                          int L, void* stream) {
+  return filter_grad_call(u, dy, dk, work, work_bytes, B, H, L, 0, stream);
+}
+
+int sffft_filter_grad_bf16(const uint16_t* u, const uint16_t* dy, float* dk, void* work, size_t work_bytes, int B,
+                           int H, int L, void* stream) {
+  return filter_grad_call(u, dy, dk, work, work_bytes, B, H, L, 1, stream);
+}
 
 size_t sffft_fft_work_bytes(int batch, int N) {
   xf::Seqs q;

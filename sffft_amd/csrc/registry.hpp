@@ -48,4 +48,11 @@ struct LongEntry {
 // Defined by long_inst.hip.
 const LongEntry* long_entries(int* n);
 
+// Defined by filter_grad.hip: the parts a call leaves to be summed (its workspace holds that many
+// [H][L] fp32 arrays when there are several; 0: not a compiled length), and the launch (io: 0 =
+// fp32, 1 = bf16).
+int filter_grad_parts(int B, int H, int L);
+hipError_t filter_grad(const void* u, const void* dy, float* dk, void* work, int B, int H, int L, int io,
+                       hipStream_t stream);
+
 }  // namespace sffft

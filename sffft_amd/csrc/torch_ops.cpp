@@ -6,6 +6,7 @@
 //   sffft::spectrum(Tensor k, int[] plan, bool conj=False) -> Tensor
 //                                    k [H, L] fp32 -> [H, 2L] complex64 (conj: its conjugate)
 //   sffft::conv(Tensor u, Tensor kf, int[] plan) -> Tensor  u [B, H, L] fp32 or bf16
+//   sffft::filter_grad(Tensor u, Tensor dy) -> Tensor  the filter's gradient [H, L] fp32
 //
 // `plan` is the nine sffft_plan fields (r0, r1, r2, waves, acc, cached, seqs, mode, channels).
 // Each operator launches on the current stream of its input's device, so it is ordered with
@@ -103,6 +104,33 @@ at::Tensor conv_gpu(const at::Tensor& u_in, const at::Tensor& kf, c10::IntArrayR
   return y;
 }
 
+// dk[h, j] = sum_b sum_{n >= j} dy[b, h, n] u[b, h, n - j], fp32 [H, L]
+at::Tensor filter_grad_gpu(const at::Tensor& u_in, const at::Tensor& dy_in) {
+  TORCH_CHECK(u_in.is_cuda() && u_in.dim() == 3 && dy_in.sizes() == u_in.sizes() && dy_in.device() == u_in.device(),
+              "sffft::filter_grad: u and dy must be [B, H, L] tensors of one shape on one GPU, got ", u_in.sizes(),
+              " and ", dy_in.sizes());
+  TORCH_CHECK((u_in.scalar_type() == at::kFloat || u_in.scalar_type() == at::kBFloat16) &&
+                  dy_in.scalar_type() == u_in.scalar_type(),
+              "sffft::filter_grad: u and dy must both be float32 or both bfloat16");
+  const c10::DeviceGuard guard(u_in.device());
+  const at::Tensor u = u_in.contiguous(), dy = dy_in.contiguous();
+  const int64_t B = u.size(0), H = u.size(1), L = u.size(2);
+  TORCH_CHECK(B <= INT32_MAX && H <= INT32_MAX && L <= INT32_MAX, "sffft::filter_grad: shape too large");
+  at::Tensor dk = at::empty({H, L}, u.options().dtype(at::kFloat));
+  const size_t wb = sffft_filter_grad_work_bytes((int)B, (int)H, (int)L);
+  at::Tensor work;
+  if (wb) work = at::empty({(int64_t)wb}, u.options().dtype(at::kByte));
+  void* w = wb ? work.data_ptr() : nullptr;
+  check(u.scalar_type() == at::kBFloat16
+            ? sffft_filter_grad_bf16(reinterpret_cast<const uint16_t*>(u.data_ptr()),
+                                     reinterpret_cast<const uint16_t*>(dy.data_ptr()), dk.data_ptr<float>(), w, wb,
+                                     (int)B, (int)H, (int)L, current_stream())
+            : sffft_filter_grad_f32(u.data_ptr<float>(), dy.data_ptr<float>(), dk.data_ptr<float>(), w, wb, (int)B,
+                                    (int)H, (int)L, current_stream()),
+        "sffft_filter_grad");
+  return dk;
+}
+
 at::Tensor call_conv(const at::Tensor& u, const at::Tensor& kf, c10::IntArrayRef plan) {
   static const auto op = c10::Dispatcher::singleton()
                              .findSchemaOrThrow("sffft::conv", "")
@@ -163,12 +191,14 @@ at::Tensor spectrum_autograd(const at::Tensor& k, c10::IntArrayRef plan, bool co
 TORCH_LIBRARY(sffft, m) {
   m.def("spectrum(Tensor k, int[] plan, bool conj=False) -> Tensor");
   m.def("conv(Tensor u, Tensor kf, int[] plan) -> Tensor");
+  m.def("filter_grad(Tensor u, Tensor dy) -> Tensor");
 }
 
 // torch names its GPU dispatch key CUDA on every backend, this one included.
 TORCH_LIBRARY_IMPL(sffft, CUDA, m) {
   m.impl("spectrum", &spectrum_gpu);
   m.impl("conv", &conv_gpu);
+  m.impl("filter_grad", &filter_grad_gpu);
 }
 
 TORCH_LIBRARY_IMPL(sffft, Autograd, m) {

@@ -37,7 +37,7 @@ from typing import List, Optional
 
 import torch
 
-from . import LONG_DEFAULT_PLANS, Plan, default_plan
+from . import LENGTHS, LONG_DEFAULT_PLANS, Plan, default_plan
 
 PLAN_FIELDS = ("r0", "r1", "r2", "waves", "acc", "cached", "seqs", "mode", "channels")
 
@@ -68,17 +68,32 @@ def _conv_fake(u, kf, plan):
     return torch.empty_like(u)
 
 
+@torch.library.register_fake("sffft::filter_grad")
+def _filter_grad_fake(u, dy):
+    torch._check(u.dim() == 3 and dy.shape == u.shape, lambda: "u and dy must be [B, H, L]")
+    return u.new_empty((u.shape[1], u.shape[2]), dtype=torch.float32)
+
+
 def filter_grad(u: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
     """dk[h, j] = sum_b sum_{n >= j} dy[b, h, n] u[b, h, n - j] for u, dy [B, H, L] (fp32 [H, L]).
 
-    Computed on the GPU kernels per sequence as the convolution of dy with the conjugate
-    spectrum of u (the correlation of the two; the conjugation is folded into the spectrum's
-    gather), summed over b: the B*H rows of u are the filters (fp32 spectra) of a
-    batch-of-one convolution. Multi-pass lengths (L > 16384) take
-    pairs of sequences only, so there each row of dy is paired with a zero row (a batch of two
-    whose second row is discarded).
+    Up to L = 16384 one fused kernel (``torch.ops.sffft.filter_grad``), which sums the batch's
+    spectra before a channel's one inverse transform. It records no gradient, so a dy whose own
+    gradient is being recorded (a second derivative) takes the composition of the differentiable
+    operators below, as the multi-pass lengths (L > 16384) do.
+
+    The composition computes per sequence the convolution of dy with the conjugate spectrum of u
+    (the correlation of the two; the conjugation is folded into the spectrum's gather), summed
+    over b: the B*H rows of u are the filters (fp32 spectra) of a batch-of-one convolution.
+    Multi-pass lengths take pairs of sequences only, so there each row of dy is paired with a zero
+    row (a batch of two whose second row is discarded).
     """
     B, H, L = u.shape
+    if L in LENGTHS and not (torch.is_grad_enabled() and dy.requires_grad):
+        u = u.detach()
+        if not u.dtype == dy.dtype == torch.bfloat16:
+            u, dy = u.float(), dy.float()
+        return torch.ops.sffft.filter_grad(u, dy.reshape(B, H, L))
     pairs_only = L in LONG_DEFAULT_PLANS
     plan = default_plan(L, "fp32", 2 if pairs_only else 1)  # one sequence per transform: batch of one
     fields = plan_fields(plan)

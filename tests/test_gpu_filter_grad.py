@@ -1,0 +1,108 @@
+"""The fused filter gradient (sffft_filter_grad_*, torch.ops.sffft.filter_grad).
+
+dk[h, j] = sum_b sum_{n >= j} dy[b, h, n] u[b, h, n - j] against an fp64 FFT correlation, at
+every compiled length (teams within one wavefront, teams of several, both halves in a workgroup
+or in the grid) and at batches and channel counts that leave a pair, a subset of the batch, a
+channel slot or a batch split partly empty.
+"""
+import ctypes
+
+import pytest
+import torch
+
+import sffft_amd as sf
+from sffft_amd import torch_ops
+
+
+def reference(u, dy):
+    L = u.shape[-1]
+    U, D = (torch.fft.rfft(x.double().cpu(), 2 * L) for x in (u, dy))
+    return torch.fft.irfft((D * U.conj()).sum(0), 2 * L)[..., :L]
+
+
+def test_argument_errors_need_no_gpu():
+    lib = sf.lib()
+    E = sf.SFFFT_EINVAL
+    null = ctypes.c_void_p(0)
+    u, dy, dk, w = (ctypes.c_void_p((1 << 40) + i * (1 << 34)) for i in range(4))
+    # one half per workgroup from L = 4096 on: two parts to sum, and a workspace for them
+    assert lib.sffft_filter_grad_work_bytes(8, 768, 1024) == 0
+    need = lib.sffft_filter_grad_work_bytes(8, 768, 4096)
+    assert need == 2 * 768 * 4096 * 4
+    assert lib.sffft_filter_grad_work_bytes(8, 768, 1000) == lib.sffft_filter_grad_work_bytes(8, 0, 4096) == 0
+    f = lib.sffft_filter_grad_f32
+    assert f(null, dy, dk, w, need, 8, 768, 4096, null) == E
+    assert f(u, dy, dk, w, need, 0, 768, 4096, null) == E
+    assert f(u, dy, dk, w, need, 8, 768, 1000, null) == E
+    assert f(u, dy, dk, w, need, 8, 768, 32768, null) == E                     # multi-pass lengths: not here
+    assert f(u, dy, dk, null, 0, 8, 768, 4096, null) == E                      # workspace missing
+    assert f(u, dy, dk, w, need - 4, 8, 768, 4096, null) == E                  # too small
+    assert f(u, dy, u, w, need, 8, 768, 4096, null) == E                       # dk overlaps u
+    assert f(u, dy, dk, dy, need, 8, 768, 4096, null) == E                     # workspace overlaps dy
+    assert f(u, dy, ctypes.c_void_p((1 << 40) + (1 << 36) + 4), w, need, 8, 768, 4096, null) == E  # dk misaligned
+    assert f(ctypes.c_void_p((1 << 40) + 2), dy, dk, w, need, 8, 768, 4096, null) == E
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("io", ["fp32", "bf16"])
+@pytest.mark.parametrize("L", sf.LENGTHS)
+def test_matches_fp64(dev, L, io):
+    g = torch.Generator(device=dev).manual_seed(L)
+    for B, H in ((1, 1), (2, 5), (3, 2), (9, 7), (16, 3)):
+        print(f"filter_grad B={B} H={H} L={L} {io}", flush=True)
+        u, dy = (torch.randn(B, H, L, device=dev, generator=g).to(torch.bfloat16 if io == "bf16" else torch.float32)
+                 for _ in range(2))
+        dk = torch.ops.sffft.filter_grad(u, dy)
+        ref = reference(u, dy)
+        err = ((dk.double().cpu() - ref).norm(dim=1) / ref.norm(dim=1)).max().item()
+        # fp32 transforms: three passes (u, dy, inverse) of at most four radix-16 stages, each with
+        # about 8 roundings of 2^-24 on the way of a value: rms 2^-24 sqrt(3 * 4 * 8) = 6e-7, and
+        # a factor of 3 for the worst channel
+        assert err <= 2e-6, (B, H, err)
+        assert torch.equal(dk, torch.ops.sffft.filter_grad(u, dy))
+
+
+@pytest.mark.gpu
+def test_any_alignment_and_stride(dev):
+    """Rows at any element offset, and non-contiguous operands, as the composed path took them."""
+    x = torch.randn(4 * 3 * 512 + 1, device=dev)
+    u, dy = x[1:].view(4, 3, 512), x[:-1].view(4, 512, 3).transpose(1, 2)
+    ref = reference(u, dy)
+    assert ((torch_ops.filter_grad(u, dy).double().cpu() - ref).norm() / ref.norm()).item() <= 2e-6
+    # an expanded output gradient, as sum().backward() makes
+    one = torch.ones((), device=dev).expand(4, 3, 512)
+    ref = reference(u, one)
+    assert ((torch_ops.filter_grad(u, one).double().cpu() - ref).norm() / ref.norm()).item() <= 2e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L", [128, 512, 1024, 4096])
+def test_race_check_build_agrees(dev, L):
+    """Bit-identical to the build whose wavefront-level LDS hand-offs are real waits."""
+    B, H = 8, 64
+    u, dy = (torch.randn(B, H, L, device=dev) for _ in range(2))
+    out = []
+    for lib in (sf.lib(), sf.load_library(sf.DEBUG_LIB_PATH)):
+        dk = torch.empty(H, L, device=dev)
+        wb = lib.sffft_filter_grad_work_bytes(B, H, L)
+        work = torch.empty(max(wb, 16), dtype=torch.uint8, device=dev)
+        p = [ctypes.c_void_p(t.data_ptr()) for t in (u, dy, dk, work)]
+        s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        assert lib.sffft_filter_grad_f32(*p, wb, B, H, L, s) == 0
+        torch.cuda.synchronize()
+        out.append(dk)
+    assert torch.equal(*out)
+
+
+@pytest.mark.gpu
+def test_second_derivative_takes_the_composed_path(dev):
+    """With the gradient's own gradient recorded, d(dk)/d(dy) is still there."""
+    u, k = torch.randn(2, 3, 256, device=dev), torch.randn(3, 256, device=dev, requires_grad=True)
+    dy = torch.randn(2, 3, 256, device=dev, requires_grad=True)
+    (dk,) = torch.autograd.grad(torch_ops.LongConv()(u, k), k, dy, create_graph=True)
+    c = torch.randn(3, 256, device=dev)
+    (g,) = torch.autograd.grad((dk * c).sum(), dy)
+    # d/d(dy) of sum_j c[h, j] dk[h, j]: the causal convolution of u with c
+    U, C = torch.fft.rfft(u.double(), 512), torch.fft.rfft(c.double(), 512)
+    ref = torch.fft.irfft(U * C, 512)[..., :256]
+    assert ((g.double() - ref).norm() / ref.norm()).item() <= 5e-4
