@@ -17,6 +17,7 @@
 #include "fftconv_wave.hpp"
 #include "longconv.hpp"
 #include "registry.hpp"
+#include "spectrum.hpp"
 #include "transforms.hpp"
 
 // Workspace of sffft_spectrum_noalloc, the one entry point that allocates nothing: a
@@ -548,12 +549,21 @@ int permute_launch(const float2* src, float2* kf, int H, const sffft_plan* plan,
   return hip_status(hipGetLastError(), "spectrum permute launch");
 }
 
+// The order of a plan's spectra (`whole`: of a complex filter; conj: conjugate spectra).
+SpectrumOrder spectrum_order(const sffft_plan* p, int whole, int conj) {
+  auto lg = [](int r) { int l = 0; while ((1 << l) < r) l++; return l; };
+  const float sc = last_stage_scale(p);
+  return {p->mode, p->mode == 1 && !whole, lg(p->r0), lg(p->r1), lg(p->r2), sc, conj ? -sc : sc};
+}
+
 // Spectrum of the H filter rows from channel h0 on: kr, plus
 // i ki for a complex filter (ki non-null, whole spectrum); with conj, its conjugate (the
-// spectrum the correlations of the backward passes run on). The padded rows are transformed
-// in place in `work` (H * N complex64; fp64 stages, complex64 between them), then gathered
-// into kernel order. Up to 16384 points the transform is one pass through LDS and needs no
-// workspace. Longer rows take the two-pass transform, whose workspace is this call's own rows
+// spectrum the correlations of the backward passes run on). Zero-padded rows of up to 16384
+// points take one launch (spectrum.hpp), which leaves `work` alone: the three launches below took
+// 36.9, 122 and 188 us where it takes 10.8, 30 and 65 (H = 768, L = 1024, 4096, 8192), with the
+// same bits. Longer rows do not fit a workgroup's LDS; they, and the unpadded ones of a circular
+// convolution, are padded into `work` (H * N complex64), transformed there in place (fp64
+// stages, complex64 between them) and gathered into kernel order. Above 16384 points that is the two-pass transform, whose workspace is this call's own rows
 // of kf: the gather overwrites them afterwards, and the results of earlier calls (the rows
 // of the channels before h0) lie before them.
 int spectrum_impl(const float* kr, const float* ki, int H, int L, int klen, const sffft_plan* plan, void* kf,
@@ -561,6 +571,16 @@ int spectrum_impl(const float* kr, const float* ki, int H, int L, int klen, cons
   if (!kr || !kf || !work || H < 1 || kf == work) return SFFFT_EINVAL;
   const int rc = check_shape(L, plan);
   if (rc) return rc;
+  // (a kf that overlaps the filter, or is aligned to 8 bytes only, takes the staged launches)
+  const uintptr_t k0 = (uintptr_t)kr, k1 = (uintptr_t)(ki ? ki : kr), f0 = (uintptr_t)kf;
+  const size_t kbytes = (size_t)(h0 + H) * klen * 4, fbytes = (size_t)(h0 + H) * 2 * L * 8;
+  const bool apart = (k0 + kbytes <= f0 || f0 + fbytes <= k0) && (k1 + kbytes <= f0 || f0 + fbytes <= k1);
+  if (klen == L && 2 * L <= SPECTRUM_ROWS_MAX_N && aligned16(kf) && apart) {
+    const size_t at = (size_t)h0 * L;
+    if (run_spectrum_rows(kr + at, ki ? ki + at : nullptr, static_cast<float4*>(kf) + at, H, 2 * L,
+                          spectrum_order(plan, whole, conj), (hipStream_t)stream))
+      return hip_status(hipGetLastError(), "spectrum launch");
+  }
   const int N = 2 * L;
   hipStream_t s = (hipStream_t)stream;
   float2* w = static_cast<float2*>(work);
