@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "../../include/sffft.h"
+#include "conv2d.hpp"
 #include "fftconv.hpp"
 #include "fftconv_wave.hpp"
 #include "longconv.hpp"
@@ -943,7 +944,9 @@ int sffft_circconv2d_f32(const float* u, const float* k, float* y, void* work, s
   if (work_bytes < need || span_overlap(work, need, u, io) || span_overlap(work, need, y, io) ||
       span_overlap(work, need, k, kb) || span_overlap(y, io, u, io) || span_overlap(y, io, k, kb))
     return SFFFT_EINVAL;
-  return hip_status(xf::circconv2d(u, k, y, static_cast<float2*>(work), B, H, N0, N1, (hipStream_t)stream),
+  float2* ws = static_cast<float2*>(work);
+  return hip_status(xf::c2::takes(N0, N1) ? xf::c2::run(u, k, y, ws, B, H, N0, N1, (hipStream_t)stream)
+                                          : xf::circconv2d(u, k, y, ws, B, H, N0, N1, (hipStream_t)stream),
                     "circconv2d launch");
 }
 
