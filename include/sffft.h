@@ -11,7 +11,7 @@
  *    u and y are [B][H][L] row-major; k is [H][L]; rows must be 16-byte aligned.
  *  - `stream` is a hipStream_t (NULL = default stream). Calls are asynchronous on
  *    that stream, reentrant, and allocate no memory, except that the first call on a
- *    device uploads an immutable 57,344-byte DFT coefficient table, and the first
+ *    device uploads an immutable 57,344-byte DFT coefficient table and its conjugate, and the first
  *    mode-1 call of a plan its twiddle table (kept for the life of the process).
  *  - Every function returns SFFFT_OK (0) or a positive error code; nothing exits.
  */
@@ -44,7 +44,7 @@ extern "C" {
  *           1 = one wavefront per transform, stages chained in registers, `waves`
  *               wavefronts per workgroup sharing LDS-resident DFT and twiddle tables
  *               (two-stage plans, seqs = 2; the first call for such a plan on a device
- *               uploads its immutable twiddle tables, 32*L bytes; 16*L for acc = 1)
+ *               uploads its immutable twiddle tables and their conjugates, 64*L bytes; 32*L for acc = 1)
  *   channels : mode 1 only: channels per workgroup; their spectra are copied into
  *           LDS once and shared by the wavefronts of each channel (mode 0: 1)
  *   mode 2 : multi-pass (sffft_conv_long_*): N = r0 * (r1 * r2), a column transform of
@@ -102,6 +102,20 @@ int sffft_spectrum(const float* k, int H, int L, const sffft_plan* plan, void* k
  * anti-causal correlation z[m] = sum_{n>=m} x[n] k[n-m] (m < L), which the input and filter
  * gradients are, is sffft_conv_* of x with this spectrum: no time reversal of x or z. */
 int sffft_spectrum_conj(const float* k, int H, int L, const sffft_plan* plan, void* kf, void* work, void* stream);
+
+/* The anti-causal correlation y[b,h,m] = sum_{n>=m} u[b,h,n] k[h,n-m], m < L, with the spectrum of
+ * sffft_spectrum (of the real filter itself, not its conjugate): the gradient of sffft_conv_* with
+ * respect to u. Arguments, alignment and workspace as for sffft_conv_* (plan modes 0 and 1) and
+ * sffft_conv_long_* (mode 2). Plans with in-kernel DFT matrices (cached = 0) return SFFFT_ENOPLAN:
+ * run sffft_conv_* with the spectrum of sffft_spectrum_conj there. No counterpart in the
+ * reference. */
+int sffft_corr_f32(const float* u, const void* kf, float* y, int B, int H, int L, const sffft_plan* plan, void* stream);
+int sffft_corr_bf16(const uint16_t* u, const void* kf, uint16_t* y, int B, int H, int L, const sffft_plan* plan,
+                    void* stream);
+int sffft_corr_long_f32(const float* u, const void* kf, float* y, void* work, size_t work_bytes, int B, int H, int L,
+                        const sffft_plan* plan, void* stream);
+int sffft_corr_long_bf16(const uint16_t* u, const void* kf, uint16_t* y, void* work, size_t work_bytes, int B, int H,
+                         int L, const sffft_plan* plan, void* stream);
 
 /* Filter gradient of the causal convolution,
  *   dk[h,j] = sum_b sum_{n>=j} dy[b,h,n] u[b,h,n-j],  j < L,

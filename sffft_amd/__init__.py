@@ -118,6 +118,10 @@ def load_library(path: str) -> ctypes.CDLL:
         "sffft_spectrum_noalloc": (ci, [vp, ci, ci, P, vp, vp]),
         "sffft_conv_f32": (ci, [vp, vp, vp, ci, ci, ci, P, vp]),
         "sffft_conv_bf16": (ci, [vp, vp, vp, ci, ci, ci, P, vp]),
+        "sffft_corr_f32": (ci, [vp, vp, vp, ci, ci, ci, P, vp]),
+        "sffft_corr_bf16": (ci, [vp, vp, vp, ci, ci, ci, P, vp]),
+        "sffft_corr_long_f32": (ci, [vp, vp, vp, vp, sz, ci, ci, ci, P, vp]),
+        "sffft_corr_long_bf16": (ci, [vp, vp, vp, vp, sz, ci, ci, ci, P, vp]),
         "sffft_conv_complex_f32": (ci, [vp, vp, vp, ci, ci, ci, P, vp]),
         "sffft_conv_complex_bf16": (ci, [vp, vp, vp, ci, ci, ci, P, vp]),
         "sffft_work_bytes": (sz, [ci, ci, ci, P]),

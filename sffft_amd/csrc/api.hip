@@ -138,13 +138,14 @@ const Entry* find_entry(int L, const sffft_plan* p) {
 // ---- DFT coefficient table (the "cached" DFT matrices, src/sffft.cu:349-362) ----
 // Entries are __float2half((float)cos(angle)) / (float)-sin(angle) of the exact
 // angle 2*pi*(e mod R)/R, as in the reference table, arranged as MFMA fragments.
-void build_table(std::vector<_Float16>& t) {
+// conj: the table of the conjugates (sines negated).
+void build_table(std::vector<_Float16>& t, bool conj) {
   t.assign((size_t)FTAB_H8 * 8, (_Float16)0.f);
   const double two_pi = 6.283185307179586476925286766559;
   auto cs = [&](int e, int R, float* c, float* s) {
     const double a = two_pi * (double)(e % R) / (double)R;
     *c = (float)std::cos(a);
-    *s = (float)std::sin(a);
+    *s = (float)(conj ? -std::sin(a) : std::sin(a));
   };
   for (int R : {16, 32, 64}) {
     const int T = R / 16;
@@ -179,15 +180,20 @@ void build_table(std::vector<_Float16>& t) {
 std::mutex g_table_mu;
 void* g_table[256];
 
-int device_table(const void** out) {
+// The device's coefficient table, or with conj the one of the conjugates, which follows it: both
+// are made by the first call, so that a capture whose eager warm-up ran only one direction finds
+// the other.
+int device_table(const void** out, int conj = 0) {
   int dev = 0;
   hipError_t err = hipGetDevice(&dev);
   if (err != hipSuccess) return hip_status(err, "hipGetDevice");
   if (dev < 0 || dev >= 256) return SFFFT_EINVAL;
   std::lock_guard<std::mutex> lock(g_table_mu);
   if (!g_table[dev]) {
-    std::vector<_Float16> host;
-    build_table(host);
+    std::vector<_Float16> host, host_conj;
+    build_table(host, false);
+    build_table(host_conj, true);
+    host.insert(host.end(), host_conj.begin(), host_conj.end());
     void* d = nullptr;
     if ((err = hipMalloc(&d, host.size() * sizeof(_Float16))) != hipSuccess) return hip_status(err, "hipMalloc");
     if ((err = hipMemcpy(d, host.data(), host.size() * sizeof(_Float16), hipMemcpyHostToDevice)) != hipSuccess) {
@@ -196,7 +202,7 @@ int device_table(const void** out) {
     }
     g_table[dev] = d;
   }
-  *out = g_table[dev];
+  *out = static_cast<const char*>(g_table[dev]) + (conj ? (size_t)FTAB_H8 * 16 : 0);
   return SFFFT_OK;
 }
 
@@ -280,8 +286,9 @@ int scratch_for_device(void** out) {
 std::mutex g_tw_mu;
 std::map<std::tuple<int, int, int>, void*> g_tw[256];  // per device: (r0, r1, layout) -> table
 
-// Twiddle tables of plan r0 x r1 in `layout`: 0 paired (fp32), 1 split (fp32), 2 fp16.
-int device_twiddles(int r0, int r1, int layout, const void** out) {
+// Twiddle tables of plan r0 x r1 in `layout`: 0 paired (fp32), 1 split (fp32), 2 fp16; with conj the
+// tables of the conjugates, which follow them.
+int device_twiddles(int r0, int r1, int layout, const void** out, int conj = 0) {
   int dev = 0;
   hipError_t err = hipGetDevice(&dev);
   if (err != hipSuccess) return hip_status(err, "hipGetDevice");
@@ -295,6 +302,10 @@ int device_twiddles(int r0, int r1, int layout, const void** out) {
       build_twiddles_h(r0, r1, host16);
     else
       build_twiddles(r0, r1, layout == 1, host32);
+    // the conjugates: imaginary parts negated (layout 2: the last four of each eight values)
+    const size_t n32 = host32.size(), n16 = host16.size();
+    for (size_t i = 0; i < n32; i++) host32.push_back(i & 1 ? -host32[i] : host32[i]);
+    for (size_t i = 0; i < n16; i++) host16.push_back(i & 4 ? -host16[i] : host16[i]);
     const void* src = layout == 2 ? (const void*)host16.data() : (const void*)host32.data();
     const size_t bytes = layout == 2 ? host16.size() * sizeof(_Float16) : host32.size() * sizeof(float);
     void* d = nullptr;
@@ -305,7 +316,7 @@ int device_twiddles(int r0, int r1, int layout, const void** out) {
     }
     slot = d;
   }
-  *out = slot;
+  *out = static_cast<const char*>(slot) + (conj ? (size_t)r0 * r1 * (layout == 2 ? 8 : 16) : 0);
   return SFFFT_OK;
 }
 
@@ -451,9 +462,10 @@ __global__ void empty_dispatch_kernel() {}
 
 // cplx: complex filters (whole spectra from sffft_spectrum_complex); wave plans then run
 // their non-Hermitian instantiation, the other plans read whole spectra anyway.
+// corr: the anti-causal correlation with the same (real) filters.
 template <int IO>
 int conv(const void* u, const void* kf, void* y, int B, int H, int L, const sffft_plan* p, void* stream,
-         int cplx = 0) {
+         int cplx = 0, int corr = 0) {
   if (!u || !kf || !y || B < 1 || H < 1 || (long long)B * H > INT_MAX) return SFFFT_EINVAL;
   int rc = check_shape(L, p);
   if (rc) return rc;
@@ -462,15 +474,17 @@ int conv(const void* u, const void* kf, void* y, int B, int H, int L, const sfff
   if (!aligned16(u) || !aligned16(y) || !aligned16(kf)) return SFFFT_EINVAL;
   const Entry* e = find_entry(L, p);
   if (!e) return SFFFT_ENOPLAN;
+  if (corr && !p->cached) return SFFFT_ENOPLAN;  // in-kernel DFT fragments: the forward ones only
   const void* table = nullptr;
-  if ((rc = device_table(&table))) return rc;
+  if ((rc = device_table(&table, corr))) return rc;
   const void* tw = nullptr;
   // wave plans: the fp16 tables for the fp16-products kernels (the fp16-accumulation
   // mode, real filters), else the fp32 tables in the plan's layout
   const bool hp = e->mode == 1 && !cplx && p->acc;
-  if (e->mode == 1 && (rc = device_twiddles(p->r0, p->r1, hp ? 2 : tw_split(p->r0, p->r1) ? 1 : 0, &tw))) return rc;
+  if (e->mode == 1 && (rc = device_twiddles(p->r0, p->r1, hp ? 2 : tw_split(p->r0, p->r1) ? 1 : 0, &tw, corr)))
+    return rc;
   const launch_fn fn = cplx && e->mode == 1 ? e->launch_complex[IO][p->cached] : e->launch[IO][p->cached];
-  return hip_status(fn(u, kf, y, B, H, table, tw, p->acc, (hipStream_t)stream), "fused convolution launch");
+  return hip_status(fn(u, kf, y, B, H, table, tw, p->acc, corr, (hipStream_t)stream), "fused convolution launch");
 }
 
 // Workspace of one channel (its B/2 pairs of 2L complex fp16 points); a workspace of
@@ -489,7 +503,7 @@ size_t work_bytes(int B, int H, int L) {
 // circ: circular convolution of period 2L (rows of length 2L)
 template <int IO>
 int conv_long(const void* u, const void* kf, void* y, void* work, size_t wbytes, int B, int H, int L,
-              const sffft_plan* p, void* stream, int circ = 0) {
+              const sffft_plan* p, void* stream, int circ = 0, int corr = 0) {
   if (!u || !kf || !y || !work || B < 2 || H < 1 || (long long)B * H > INT_MAX) return SFFFT_EINVAL;
   int rc = check_shape(L, p);
   if (rc) return rc;
@@ -514,10 +528,10 @@ int conv_long(const void* u, const void* kf, void* y, void* work, size_t wbytes,
   const LongEntry* e = find_long_entry(p);
   if (!e) return SFFFT_ENOPLAN;
   const void* table = nullptr;
-  if ((rc = device_table(&table))) return rc;
+  if ((rc = device_table(&table, corr))) return rc;
   const void* tw = nullptr;
-  if ((rc = device_twiddles(p->r1, p->r2, 0, &tw))) return rc;
-  return hip_status(e->launch[circ][IO](u, kf, y, work, B, H, chunk, table, tw, (hipStream_t)stream),
+  if ((rc = device_twiddles(p->r1, p->r2, 0, &tw, corr))) return rc;
+  return hip_status(e->launch[circ][IO](u, kf, y, work, B, H, chunk, table, tw, corr, (hipStream_t)stream),
                     "multi-pass launch");
 }
 
@@ -750,6 +764,26 @@ int sffft_conv_f32(const float* u, const void* kf, float* y, int B, int H, int L
 int sffft_conv_bf16(const uint16_t* u, const void* kf, uint16_t* y, int B, int H, int L, const sffft_plan* plan,
                     void* stream) {
   return conv<1>(u, kf, y, B, H, L, plan, stream);
+}
+
+int sffft_corr_f32(const float* u, const void* kf, float* y, int B, int H, int L, const sffft_plan* plan,
+                   void* stream) {
+  return conv<0>(u, kf, y, B, H, L, plan, stream, 0, 1);
+}
+
+int sffft_corr_bf16(const uint16_t* u, const void* kf, uint16_t* y, int B, int H, int L, const sffft_plan* plan,
+                    void* stream) {
+  return conv<1>(u, kf, y, B, H, L, plan, stream, 0, 1);
+}
+
+int sffft_corr_long_f32(const float* u, const void* kf, float* y, void* work, size_t work_bytes, int B, int H, int L,
+                        const sffft_plan* plan, void* stream) {
+  return conv_long<0>(u, kf, y, work, work_bytes, B, H, L, plan, stream, 0, 1);
+}
+
+int sffft_corr_long_bf16(const uint16_t* u, const void* kf, uint16_t* y, void* work, size_t work_bytes, int B, int H,
+                         int L, const sffft_plan* plan, void* stream) {
+  return conv_long<1>(u, kf, y, work, work_bytes, B, H, L, plan, stream, 0, 1);
 }
 
 int sffft_conv_complex_f32(const float* u, const void* kf, float* y, int B, int H, int L, const sffft_plan* plan,

@@ -23,23 +23,24 @@ constexpr int fused_wpe() {
 
 template <class P, int NW, int NSEQ, class TIO, bool CACHED>
 static hipError_t launch_fused(const void* u, const void* kf, void* y, int B, int H, const void* ftab, const void*,
-                               int acc16, hipStream_t stream) {
+                               int acc16, int corr, hipStream_t stream) {
   const unsigned grid = (unsigned)(H * (B / NSEQ));
   constexpr int WPE = fused_wpe<P, NW, CACHED>();
+  const float inv_n = (corr ? -1.f : 1.f) / (float)P::N;  // exact: N is a power of two
   if (acc16)
     hipLaunchKernelGGL((fftconv_kernel<P, NW, NSEQ, TIO, CACHED, true, WPE>), dim3(grid), dim3(64 * NW), 0, stream,
                        static_cast<const TIO*>(u), static_cast<const float2*>(kf), static_cast<TIO*>(y), B, H,
-                       static_cast<const h8*>(ftab));
+                       static_cast<const h8*>(ftab), inv_n);
   else
     hipLaunchKernelGGL((fftconv_kernel<P, NW, NSEQ, TIO, CACHED, false, WPE>), dim3(grid), dim3(64 * NW), 0, stream,
                        static_cast<const TIO*>(u), static_cast<const float2*>(kf), static_cast<TIO*>(y), B, H,
-                       static_cast<const h8*>(ftab));
+                       static_cast<const h8*>(ftab), inv_n);
   return hipGetLastError();
 }
 
 template <class P, int NW, int CH, class TIO, bool CACHED>
 static hipError_t launch_wave(const void* u, const void* kf, void* y, int B, int H, const void* ftab,
-                              const void* tw, int acc16, hipStream_t stream) {
+                              const void* tw, int acc16, int, hipStream_t stream) {
   const unsigned grid = (unsigned)((H + CH - 1) / CH);
   if (acc16)
     hipLaunchKernelGGL((fftconv_wave_kernel<P, NW, CH, TIO, CACHED, true, true>), dim3(grid), dim3(64 * NW), 0,
@@ -55,7 +56,7 @@ static hipError_t launch_wave(const void* u, const void* kf, void* y, int B, int
 // complex filters: whole spectra, fp32 accumulation
 template <class P, int NW, int CH, class TIO, bool CACHED>
 static hipError_t launch_wave_complex(const void* u, const void* kf, void* y, int B, int H, const void* ftab,
-                                      const void* tw, int, hipStream_t stream) {
+                                      const void* tw, int, int, hipStream_t stream) {
   const unsigned grid = (unsigned)((H + CH - 1) / CH);
   hipLaunchKernelGGL((fftconv_wave_kernel<P, NW, CH, TIO, CACHED, false, false>), dim3(grid), dim3(64 * NW), 0,
                      stream, static_cast<const TIO*>(u), static_cast<const float4*>(kf), static_cast<TIO*>(y), B, H,

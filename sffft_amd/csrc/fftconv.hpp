@@ -208,13 +208,14 @@ struct FragSet {
 
 // w[v] = sc * exp(-2*pi*i * (e0 + step*v) / N), v = 0..3 (src/sffft.cu:106-113 for the
 // exponent): the base from v_sin/v_cos with the angle reduced to (-1/2, 1/2]
-// revolutions (e/N is exact), the others by a complex recurrence.
+// revolutions (e/N is exact), the others by a complex recurrence. inv_n = -1/N gives the
+// conjugates (the anti-causal correlation: see fftconv_kernel).
 template <int N>
-__device__ __forceinline__ void twiddle4e(int e0, int step, float sc, float* wr, float* wi) {
+__device__ __forceinline__ void twiddle4e(int e0, int step, float sc, float* wr, float* wi, float inv_n = 1.0f / N) {
   e0 &= N - 1;
   step &= N - 1;
-  const float x0 = (float)(e0 > N / 2 ? e0 - N : e0) * (1.0f / N);
-  const float x1 = (float)(step > N / 2 ? step - N : step) * (1.0f / N);
+  const float x0 = (float)(e0 > N / 2 ? e0 - N : e0) * inv_n;
+  const float x1 = (float)(step > N / 2 ? step - N : step) * inv_n;
   float r = sc * cos_rev(x0), i = -sc * sin_rev(x0);
   const float sr = cos_rev(x1), si = -sin_rev(x1);
   wr[0] = r;
@@ -239,8 +240,8 @@ __device__ __forceinline__ void cmul4(float* r, float* i, const float* fr, const
 }
 // w[v] = sc * exp(-2*pi*i * a*(b0+v) / N)
 template <int N>
-__device__ __forceinline__ void twiddle4(int a, int b0, float sc, float* wr, float* wi) {
-  twiddle4e<N>(a * b0, a, sc, wr, wi);
+__device__ __forceinline__ void twiddle4(int a, int b0, float sc, float* wr, float* wi, float inv_n) {
+  twiddle4e<N>(a * b0, a, sc, wr, wi, inv_n);
 }
 
 // 8-half operand: slots 0..3 from the real plane, 4..7 from the imaginary plane.
@@ -402,8 +403,8 @@ struct P1Frags {
 
 template <class P, int NW, int NSEQ, class TIO, bool CACHED, bool SPLIT_IN>
 __device__ __forceinline__ void phase1(const P1Data<P, NW, NSEQ, TIO>& d, P1Frags<P, NW, NSEQ, CACHED>& fr,
-                                       _Float16* re, _Float16* im, const h8* __restrict__ ftab, int acc16, int lane,
-                                       int wave) {
+                                       _Float16* re, _Float16* im, const h8* __restrict__ ftab, int acc16, float inv_n,
+                                       int lane, int wave) {
   using SP = P1Split<P, NW, NSEQ>;
   constexpr int R0 = P::R0, N = P::N, KS = SP::KS, SI = SPLIT_IN ? 1 : 0;
   constexpr float sc0 = R0 == 16 ? 0.25f : R0 == 32 ? 0.17677669529663687f : 0.125f;
@@ -424,7 +425,7 @@ __device__ __forceinline__ void phase1(const P1Data<P, NW, NSEQ, TIO>& d, P1Frag
         for (int ks = 0; ks < KS; ks++)
 #pragma unroll
           for (int k = 0; k < 2; k++) asm volatile("" : "+v"(fr.f[j][ks][k]));
-        twiddle4<N>(16 * nt + r, 16 * SP::mt(wave, 0) + 4 * g, sc0, t0r[j], t0i[j]);
+        twiddle4<N>(16 * nt + r, 16 * SP::mt(wave, 0) + 4 * g, sc0, t0r[j], t0i[j], inv_n);
 #pragma unroll
         for (int v = 0; v < 4; v++) asm volatile("" : "+v"(t0r[j][v]), "+v"(t0i[j][v]));
       }
@@ -466,7 +467,7 @@ __device__ __forceinline__ void phase1(const P1Data<P, NW, NSEQ, TIO>& d, P1Frag
 #pragma unroll
           for (int v = 0; v < 4; v++) wr[v] = t0r[PF > 0 ? j : 0][v], wi[v] = t0i[PF > 0 ? j : 0][v];
         } else {
-          twiddle4<N>(k0, 16 * mt + 4 * g, sc0, wr, wi);
+          twiddle4<N>(k0, 16 * mt + 4 * g, sc0, wr, wi, inv_n);
         }
         h4 hr, hi;  // the twiddled tile in fp16
         if (acc16) {
@@ -569,7 +570,7 @@ __device__ __forceinline__ void k_prefetch_s2(const float2* __restrict__ K, KDat
 
 template <class P, int NW, bool CACHED, bool SPLIT>
 __device__ __forceinline__ void phase2_s2(_Float16* re, _Float16* im, const KData2<P, NW>& kd,
-                                          const h8* __restrict__ ftab, int acc16, int lane, int wave) {
+                                          const h8* __restrict__ ftab, int acc16, float inv_n, int lane, int wave) {
   constexpr int R0 = P::R0, R1 = P::R1, N = P::N, ST = R0 / 16, T1 = R1 / 16;
   constexpr int UPW = (ST + NW - 1) / NW;
   constexpr float sc1 = R1 == 16 ? 0.25f : R1 == 32 ? 0.17677669529663687f : 0.125f;
@@ -608,7 +609,7 @@ __device__ __forceinline__ void phase2_s2(_Float16* re, _Float16* im, const KDat
           }
         }
         float wr[4], wi[4];
-        twiddle4<N>(16 * nt + c, 16 * s + 4 * g, sc1, wr, wi);
+        twiddle4<N>(16 * nt + c, 16 * s + 4 * g, sc1, wr, wi, inv_n);
         if (acc16) {
           cmul_hp(er, ei, hw_of(wr, wi), outr[i][nt], outi[i][nt]);
         } else {
@@ -668,7 +669,7 @@ __device__ __forceinline__ void pack_operand(const float* xr, const float* xi, h
 
 template <class P, int NW, bool CACHED, int SPLITS>
 __device__ __forceinline__ void phase2_s3(_Float16* re, _Float16* im, const float2* __restrict__ K,
-                                          const h8* __restrict__ ftab, int acc16, int lane, int wave) {
+                                          const h8* __restrict__ ftab, int acc16, float inv_n, int lane, int wave) {
   constexpr int R0 = P::R0, R1 = P::R1, R2 = P::R2, N = P::N, T1 = R1 / 16, T2 = R2 / 16;
   constexpr int ROWS = R0 / NW;
   constexpr int SB = SPLITS & 1, SE = (SPLITS >> 2) & 1;
@@ -698,7 +699,7 @@ __device__ __forceinline__ void phase2_s3(_Float16* re, _Float16* im, const floa
   constexpr bool SHARED_TW = T1 == 1 && T2 == 1;
   static_assert(!SHARED_TW || sc1 == sc2, "one tile per axis: equal radices");
   float twr[4], twi[4];
-  if constexpr (SHARED_TW) twiddle4<N>(R0 * c, 4 * g, sc1, twr, twi);
+  if constexpr (SHARED_TW) twiddle4<N>(R0 * c, 4 * g, sc1, twr, twi, inv_n);
   auto tw_n1 = [&](int nt, int t2, float sc, float* wr, float* wi) {
     if constexpr (SHARED_TW) {
 #pragma unroll
@@ -707,7 +708,7 @@ __device__ __forceinline__ void phase2_s3(_Float16* re, _Float16* im, const floa
         wi[v] = twi[v];
       }
     } else {
-      twiddle4<N>(R0 * (16 * nt + c), 16 * t2 + 4 * g, sc, wr, wi);
+      twiddle4<N>(R0 * (16 * nt + c), 16 * t2 + 4 * g, sc, wr, wi, inv_n);
     }
   };
   auto twiddle = [](const f4& er, const f4& ei, const float* wr, const float* wi, float* xr, float* xi) {
@@ -776,8 +777,8 @@ __device__ __forceinline__ void phase2_s3(_Float16* re, _Float16* im, const floa
   float lr[4], li[4], fr[4], fi[4];
   if constexpr (REC) {
     const int m0 = 4 * g * R2 + c;  // lane value v: m = m0 + v R2
-    twiddle4e<N>(wave * ROWS * m0, wave * ROWS * R2, sc1, lr, li);
-    twiddle4e<N>(m0, R2, 1.f, fr, fi);
+    twiddle4e<N>(wave * ROWS * m0, wave * ROWS * R2, sc1, lr, li, inv_n);
+    twiddle4e<N>(m0, R2, 1.f, fr, fi, inv_n);
   }
   // Two forms of the same row loop. One row per step keeps the loop that the multi-tile
   // plans were tuned with: the several-row form, even with one row per step, changes how
@@ -874,7 +875,7 @@ __device__ __forceinline__ void phase2_s3(_Float16* re, _Float16* im, const floa
             for (int v = 0; v < 4; v++) wr[v] = lr[v], wi[v] = li[v];
             if (i + 1 < ROWS) cmul4(lr, li, fr, fi);
           } else {
-            twiddle4e<N>(k0 * ((16 * mt + 4 * g) * R2 + 16 * nt + c), k0 * R2, sc1, wr, wi);
+            twiddle4e<N>(k0 * ((16 * mt + 4 * g) * R2 + 16 * nt + c), k0 * R2, sc1, wr, wi, inv_n);
           }
           // back into the row's own block, [n2][n1]: only this wavefront reads the row,
           // and all of its input is in registers by now
@@ -991,7 +992,7 @@ __device__ __forceinline__ void phase2_s3(_Float16* re, _Float16* im, const floa
               for (int v = 0; v < 4; v++) wr[v] = lr[v], wi[v] = li[v];
               if (i0 + u + 1 < ROWS) cmul4(lr, li, fr, fi);
             } else {
-              twiddle4e<N>(k0[u] * ((16 * mt + 4 * g) * R2 + 16 * nt + c), k0[u] * R2, sc1, wr, wi);
+              twiddle4e<N>(k0[u] * ((16 * mt + 4 * g) * R2 + 16 * nt + c), k0[u] * R2, sc1, wr, wi, inv_n);
             }
             // back into the row's own block, [n2][n1]: only this wavefront reads the row,
             // and all of its input is in registers by now
@@ -1106,6 +1107,10 @@ constexpr int fp32_splits() {
   return SFFFT_FP32_SPLITS | (P::S == 3 && P::N == 8192 ? 4 : 0);
 }
 
+// inv_n = 1/N. With -1/N and a coefficient table of conjugates every transform is the conjugate
+// one: with F* in place of F the schedule gives conj(F*{conj(F*{z} K)}) = F{F*{z*} K*}* on z = a + i b, and
+// F*{z} = conj(F{z*}), so it is corr(a, k) + i corr(b, k), the anti-causal correlation with the
+// filter whose spectrum K is (sum_{n>=m} x[n] k[n-m]), from the convolution's own spectrum.
 // grid = H * (B / NSEQ) workgroups of 64*NW lanes; one sequence (NSEQ = 1) or one
 // pair of sequences of the same channel (NSEQ = 2) per workgroup.
 // ACC16 (fp16-accumulation mode) is a compile-time choice: as a runtime flag every
@@ -1116,7 +1121,7 @@ constexpr int fp32_splits() {
 template <class P, int NW, int NSEQ, class TIO, bool CACHED, bool ACC16, int WPE>
 __global__ void __launch_bounds__(64 * NW, WPE)
     fftconv_kernel(const TIO* __restrict__ u, const float2* __restrict__ kf, TIO* __restrict__ y, int B, int H,
-                   const h8* __restrict__ ftab) {
+                   const h8* __restrict__ ftab, float inv_n) {
   constexpr int acc16 = ACC16 ? 1 : 0;
   __shared__ __attribute__((aligned(16))) _Float16 lds[2 * P::PLANE];
   _Float16* re = lds;
@@ -1141,13 +1146,13 @@ __global__ void __launch_bounds__(64 * NW, WPE)
   if constexpr (P::S == 2) {
     KData2<P, NW> kd;
     k_prefetch_s2<P, NW>(K, kd, lane, wave);
-    phase1<P, NW, NSEQ, TIO, CACHED, SPLIT_IN>(ad, fr, re, im, ftab, acc16, lane, wave);
+    phase1<P, NW, NSEQ, TIO, CACHED, SPLIT_IN>(ad, fr, re, im, ftab, acc16, inv_n, lane, wave);
     __syncthreads();
-    phase2_s2<P, NW, CACHED, sizeof(TIO) == 4 && !ACC16>(re, im, kd, ftab, acc16, lane, wave);
+    phase2_s2<P, NW, CACHED, sizeof(TIO) == 4 && !ACC16>(re, im, kd, ftab, acc16, inv_n, lane, wave);
   } else {
-    phase1<P, NW, NSEQ, TIO, CACHED, SPLIT_IN>(ad, fr, re, im, ftab, acc16, lane, wave);
+    phase1<P, NW, NSEQ, TIO, CACHED, SPLIT_IN>(ad, fr, re, im, ftab, acc16, inv_n, lane, wave);
     __syncthreads();
-    phase2_s3<P, NW, CACHED, sizeof(TIO) == 4 && !ACC16 ? fp32_splits<P>() : 0>(re, im, K, ftab, acc16, lane, wave);
+    phase2_s3<P, NW, CACHED, sizeof(TIO) == 4 && !ACC16 ? fp32_splits<P>() : 0>(re, im, K, ftab, acc16, inv_n, lane, wave);
   }
   __syncthreads();
   phase3<P, NW, NSEQ, TIO, CACHED>(y + row_a, y + row_b, re, im, ftab, acc16, lane, wave);

@@ -39,9 +39,9 @@ static unsigned rows_grid(int nrows) {
 // chunk*(B/2) pairs of N complex fp16 points. CIRC: circular convolution of period N.
 template <int NC, int R0, int R1, class TIO, bool CIRC>
 static hipError_t launch_long(const void* u, const void* kf, void* y, void* work, int B, int H, int chunk,
-                              const void* ftab, const void* tw, hipStream_t s) {
+                              const void* ftab, const void* tw, int corr, hipStream_t s) {
   constexpr int NR = R0 * R1, N = NC * NR;
-  const float inv_n = 1.0f / (float)N;  // exact: N is a power of two
+  const float inv_n = (corr ? -1.0f : 1.0f) / (float)N;  // exact: N is a power of two; the sign conjugates
   const int BP = B / 2;
   for (int h0 = 0; h0 < H; h0 += chunk) {
     const int nch = H - h0 < chunk ? H - h0 : chunk, pi0 = h0 * BP;

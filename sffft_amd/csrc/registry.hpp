@@ -4,9 +4,10 @@
 
 namespace sffft {
 
-// Launches one instantiation. `tw` is the plan's twiddle table (wave pipeline only).
+// Launches one instantiation. `tw` is the plan's twiddle table (wave pipeline only). corr: the
+// anti-causal correlation; ftab and tw are then the tables of conjugates.
 typedef hipError_t (*launch_fn)(const void* u, const void* kf, void* y, int B, int H, const void* ftab,
-                                const void* tw, int acc16, hipStream_t stream);
+                                const void* tw, int acc16, int corr, hipStream_t stream);
 
 // One (plan, waves, sequences-per-workgroup, mode) instantiation: launchers and kernel
 // symbols for [io: 0 = fp32, 1 = bf16][cached: 0 = in-kernel DFT matrices, 1 = table].
@@ -39,7 +40,7 @@ const Entry* entries_L16384(int* n);
 // passes run on one stream with the caller's workspace.
 // `chunk` channels per group of three launches (the workspace holds chunk*B/2 pairs).
 typedef hipError_t (*long_launch_fn)(const void* u, const void* kf, void* y, void* work, int B, int H, int chunk,
-                                     const void* ftab, const void* tw, hipStream_t stream);
+                                     const void* ftab, const void* tw, int corr, hipStream_t stream);
 struct LongEntry {
   int nc, r0, r1, lds_bytes;  // lds_bytes: the row pass's tables
   long_launch_fn launch[2][2];  // [0 = causal, 1 = circular of period 2L][io: 0 = fp32, 1 = bf16]

@@ -6,7 +6,11 @@
 //   sffft::spectrum(Tensor k, int[] plan, bool conj=False) -> Tensor
 //                                    k [H, L] fp32 -> [H, 2L] complex64 (conj: its conjugate)
 //   sffft::conv(Tensor u, Tensor kf, int[] plan) -> Tensor  u [B, H, L] fp32 or bf16
+//   sffft::corr(Tensor u, Tensor kf, int[] plan) -> Tensor  the anti-causal correlation, conv's
+//                                    adjoint in u, with conv's spectrum
 //   sffft::filter_grad(Tensor u, Tensor dy) -> Tensor  the filter's gradient [H, L] fp32
+//   sffft::longconv(Tensor u, Tensor k, Tensor kf, int[] plan) -> Tensor  conv(u, kf), with
+//                                    gradients for u and for the filter k that kf was made from
 //
 // `plan` is the nine sffft_plan fields (r0, r1, r2, waves, acc, cached, seqs, mode, channels).
 // Each operator launches on the current stream of its input's device, so it is ordered with
@@ -19,11 +23,11 @@
 // used only while tracing, stay in Python (sffft_amd/torch_ops.py).
 //
 // Gradients: sffft::conv is differentiable in u. The adjoint of causal convolution is the
-// anti-causal correlation du[m] = sum_{n >= m} dy[n] k[n - m]. With the N = 2L zero padding
-// that is IDFT(DFT(dy) * conj(K))[m] for m < L: the same kernel on the conjugated spectrum
-// (elementwise conjugation of the kernel-order buffer is the kernel-order buffer of conj(K),
-// Hermitian halves included), with no time reversal of dy or du. sffft::spectrum has no
-// gradient; backpropagating through it raises.
+// anti-causal correlation du[m] = sum_{n >= m} dy[n] k[n - m], which with the N = 2L zero padding
+// is IDFT(DFT(dy) * conj(K))[m] for m < L: sffft::corr, the same kernels with conjugate DFT and
+// twiddle tables, on the same spectrum and with no time reversal of dy or du. sffft::longconv is
+// differentiable in u and in the filter. sffft::spectrum has no gradient; backpropagating through
+// it raises.
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
@@ -65,7 +69,8 @@ at::Tensor spectrum_gpu(const at::Tensor& k_in, c10::IntArrayRef plan_fields, bo
   return kf;
 }
 
-at::Tensor conv_gpu(const at::Tensor& u_in, const at::Tensor& kf, c10::IntArrayRef plan_fields) {
+at::Tensor run_conv(const at::Tensor& u_in, const at::Tensor& kf_in, c10::IntArrayRef plan_fields, bool corr) {
+  at::Tensor kf = kf_in;
   TORCH_CHECK(u_in.is_cuda() && u_in.dim() == 3, "sffft::conv: u must be a [B, H, L] GPU tensor");
   TORCH_CHECK(u_in.scalar_type() == at::kFloat || u_in.scalar_type() == at::kBFloat16,
               "sffft::conv: u must be float32 or bfloat16");
@@ -81,6 +86,10 @@ at::Tensor conv_gpu(const at::Tensor& u_in, const at::Tensor& kf, c10::IntArrayR
   TORCH_CHECK(kf.dim() == 2 && kf.size(0) == H && kf.size(1) == 2 * L, "sffft::conv: kf must be [H, 2L] = [", H,
               ", ", 2 * L, "] for u of shape ", u.sizes(), ", got ", kf.sizes());
   const sffft_plan p = to_plan(plan_fields);
+  if (corr && !p.cached) {  // in-kernel DFT fragments: no conjugate ones, so the conjugate spectrum
+    kf = at::conj_physical(kf);
+    corr = false;
+  }
   at::Tensor y = at::empty_like(u);
   const bool bf16 = u.scalar_type() == at::kBFloat16;
   void* s = current_stream();
@@ -88,20 +97,34 @@ at::Tensor conv_gpu(const at::Tensor& u_in, const at::Tensor& kf, c10::IntArrayR
     const size_t wb = sffft_work_bytes((int)B, (int)H, (int)L, &p);
     at::Tensor work = at::empty({(int64_t)std::max<size_t>(wb, 16)}, u.options().dtype(at::kByte));
     const size_t have = (size_t)work.numel();
-    check(bf16 ? sffft_conv_long_bf16(reinterpret_cast<const uint16_t*>(u.data_ptr()), kf.data_ptr(),
-                                      reinterpret_cast<uint16_t*>(y.data_ptr()), work.data_ptr(), have, (int)B,
-                                      (int)H, (int)L, &p, s)
-               : sffft_conv_long_f32(u.data_ptr<float>(), kf.data_ptr(), y.data_ptr<float>(), work.data_ptr(), have,
-                                     (int)B, (int)H, (int)L, &p, s),
+    const auto run16 = corr ? sffft_corr_long_bf16 : sffft_conv_long_bf16;
+    const auto run32 = corr ? sffft_corr_long_f32 : sffft_conv_long_f32;
+    check(bf16 ? run16(reinterpret_cast<const uint16_t*>(u.data_ptr()), kf.data_ptr(),
+                       reinterpret_cast<uint16_t*>(y.data_ptr()), work.data_ptr(), have, (int)B, (int)H, (int)L, &p, s)
+               : run32(u.data_ptr<float>(), kf.data_ptr(), y.data_ptr<float>(), work.data_ptr(), have, (int)B, (int)H,
+                       (int)L, &p, s),
           "sffft_conv_long");
   } else {
-    check(bf16 ? sffft_conv_bf16(reinterpret_cast<const uint16_t*>(u.data_ptr()), kf.data_ptr(),
-                                 reinterpret_cast<uint16_t*>(y.data_ptr()), (int)B, (int)H, (int)L, &p, s)
-               : sffft_conv_f32(u.data_ptr<float>(), kf.data_ptr(), y.data_ptr<float>(), (int)B, (int)H, (int)L, &p,
-                                s),
+    const auto run16 = corr ? sffft_corr_bf16 : sffft_conv_bf16;
+    const auto run32 = corr ? sffft_corr_f32 : sffft_conv_f32;
+    check(bf16 ? run16(reinterpret_cast<const uint16_t*>(u.data_ptr()), kf.data_ptr(),
+                       reinterpret_cast<uint16_t*>(y.data_ptr()), (int)B, (int)H, (int)L, &p, s)
+               : run32(u.data_ptr<float>(), kf.data_ptr(), y.data_ptr<float>(), (int)B, (int)H, (int)L, &p, s),
           "sffft_conv");
   }
   return y;
+}
+
+at::Tensor conv_gpu(const at::Tensor& u, const at::Tensor& kf, c10::IntArrayRef plan) {
+  return run_conv(u, kf, plan, false);
+}
+
+at::Tensor corr_gpu(const at::Tensor& u, const at::Tensor& kf, c10::IntArrayRef plan) {
+  return run_conv(u, kf, plan, true);
+}
+
+at::Tensor longconv_gpu(const at::Tensor& u, const at::Tensor&, const at::Tensor& kf, c10::IntArrayRef plan) {
+  return run_conv(u, kf, plan, false);
 }
 
 // dk[h, j] = sum_b sum_{n >= j} dy[b, h, n] u[b, h, n - j], fp32 [H, L]
@@ -138,6 +161,28 @@ at::Tensor call_conv(const at::Tensor& u, const at::Tensor& kf, c10::IntArrayRef
   return op.call(u, kf, plan);
 }
 
+at::Tensor call_corr(const at::Tensor& u, const at::Tensor& kf, c10::IntArrayRef plan) {
+  static const auto op = c10::Dispatcher::singleton()
+                             .findSchemaOrThrow("sffft::corr", "")
+                             .typed<at::Tensor(const at::Tensor&, const at::Tensor&, c10::IntArrayRef)>();
+  return op.call(u, kf, plan);
+}
+
+at::Tensor call_filter_grad(const at::Tensor& u, const at::Tensor& dy) {
+  static const auto op = c10::Dispatcher::singleton()
+                             .findSchemaOrThrow("sffft::filter_grad", "")
+                             .typed<at::Tensor(const at::Tensor&, const at::Tensor&)>();
+  return op.call(u, dy);
+}
+
+at::Tensor call_longconv(const at::Tensor& u, const at::Tensor& k, const at::Tensor& kf, c10::IntArrayRef plan) {
+  static const auto op =
+      c10::Dispatcher::singleton()
+          .findSchemaOrThrow("sffft::longconv", "")
+          .typed<at::Tensor(const at::Tensor&, const at::Tensor&, const at::Tensor&, c10::IntArrayRef)>();
+  return op.call(u, k, kf, plan);
+}
+
 at::Tensor call_spectrum(const at::Tensor& k, c10::IntArrayRef plan, bool conj) {
   static const auto op = c10::Dispatcher::singleton()
                              .findSchemaOrThrow("sffft::spectrum", "")
@@ -148,21 +193,76 @@ at::Tensor call_spectrum(const at::Tensor& k, c10::IntArrayRef plan, bool conj) 
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
-class ConvFn : public torch::autograd::Function<ConvFn> {
+// conv and corr are each other's adjoints in u.
+template <bool CORR>
+class ConvFn : public torch::autograd::Function<ConvFn<CORR>> {
  public:
   static at::Tensor forward(AutogradContext* ctx, const at::Tensor& u, const at::Tensor& kf,
                             c10::IntArrayRef plan) {
     ctx->save_for_backward({kf});
     ctx->saved_data["plan"] = plan.vec();
     at::AutoDispatchBelowADInplaceOrView guard;
-    return call_conv(u, kf, plan);
+    return CORR ? call_corr(u, kf, plan) : call_conv(u, kf, plan);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const at::Tensor kf = ctx->get_saved_variables()[0];
     const std::vector<int64_t> plan = ctx->saved_data["plan"].toIntVector();
     at::Tensor du;
-    if (ctx->needs_input_grad(0)) du = call_conv(grads[0].contiguous(), at::conj_physical(kf), plan);
+    if (ctx->needs_input_grad(0)) {
+      const at::Tensor dy = grads[0].contiguous();
+      du = CORR ? call_conv(dy, kf, plan) : call_corr(dy, kf, plan);
+    }
     return {du, at::Tensor(), at::Tensor()};
+  }
+};
+
+// The filter gradient where its own gradient is recorded (a second derivative): linear in dy, with
+// the adjoint dy' = causal_conv(u, g) for g [H, L], which longconv differentiates further. u takes no
+// gradient here.
+class FilterGradFn : public torch::autograd::Function<FilterGradFn> {
+ public:
+  static at::Tensor forward(AutogradContext* ctx, const at::Tensor& u, const at::Tensor& dy, c10::IntArrayRef plan) {
+    ctx->save_for_backward({u});
+    ctx->saved_data["plan"] = plan.vec();
+    at::AutoDispatchBelowADInplaceOrView guard;
+    return call_filter_grad(u, dy);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const at::Tensor u = ctx->get_saved_variables()[0].detach();
+    const std::vector<int64_t> plan = ctx->saved_data["plan"].toIntVector();
+    at::Tensor ddy;
+    if (ctx->needs_input_grad(1)) {
+      const at::Tensor g = grads[0].contiguous();
+      ddy = call_longconv(u, g, call_spectrum(g.detach(), plan, false), plan);
+    }
+    return {at::Tensor(), ddy, at::Tensor()};
+  }
+};
+
+// y = conv(u, kf) with gradients for u and for the filter k that kf was made from (L <= 16384).
+class LongConvFn : public torch::autograd::Function<LongConvFn> {
+ public:
+  static at::Tensor forward(AutogradContext* ctx, const at::Tensor& u, const at::Tensor& k, const at::Tensor& kf,
+                            c10::IntArrayRef plan) {
+    ctx->save_for_backward({u, kf});
+    ctx->saved_data["plan"] = plan.vec();
+    at::AutoDispatchBelowADInplaceOrView guard;
+    return call_longconv(u, k, kf, plan);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list saved = ctx->get_saved_variables();
+    const std::vector<int64_t> plan = ctx->saved_data["plan"].toIntVector();
+    const at::Tensor u = saved[0];
+    const at::Tensor dy = grads[0].to(u.scalar_type()).contiguous();
+    at::Tensor du, dk;
+    if (ctx->needs_input_grad(0)) du = call_corr(dy, saved[1], plan);
+    if (ctx->needs_input_grad(1)) {
+      if (at::GradMode::is_enabled() && dy.requires_grad())
+        dk = FilterGradFn::apply(u.detach(), dy, plan);
+      else
+        dk = call_filter_grad(u.detach(), dy);
+    }
+    return {du, dk, at::Tensor(), at::Tensor()};
   }
 };
 
@@ -179,7 +279,15 @@ class SpectrumFn : public torch::autograd::Function<SpectrumFn> {
 };
 
 at::Tensor conv_autograd(const at::Tensor& u, const at::Tensor& kf, c10::IntArrayRef plan) {
-  return ConvFn::apply(u, kf, plan);
+  return ConvFn<false>::apply(u, kf, plan);
+}
+
+at::Tensor corr_autograd(const at::Tensor& u, const at::Tensor& kf, c10::IntArrayRef plan) {
+  return ConvFn<true>::apply(u, kf, plan);
+}
+
+at::Tensor longconv_autograd(const at::Tensor& u, const at::Tensor& k, const at::Tensor& kf, c10::IntArrayRef plan) {
+  return LongConvFn::apply(u, k, kf, plan);
 }
 
 at::Tensor spectrum_autograd(const at::Tensor& k, c10::IntArrayRef plan, bool conj) {
@@ -191,6 +299,8 @@ at::Tensor spectrum_autograd(const at::Tensor& k, c10::IntArrayRef plan, bool co
 TORCH_LIBRARY(sffft, m) {
   m.def("spectrum(Tensor k, int[] plan, bool conj=False) -> Tensor");
   m.def("conv(Tensor u, Tensor kf, int[] plan) -> Tensor");
+  m.def("corr(Tensor u, Tensor kf, int[] plan) -> Tensor");
+  m.def("longconv(Tensor u, Tensor k, Tensor kf, int[] plan) -> Tensor");
   m.def("filter_grad(Tensor u, Tensor dy) -> Tensor");
 }
 
@@ -198,10 +308,14 @@ TORCH_LIBRARY(sffft, m) {
 TORCH_LIBRARY_IMPL(sffft, CUDA, m) {
   m.impl("spectrum", &spectrum_gpu);
   m.impl("conv", &conv_gpu);
+  m.impl("corr", &corr_gpu);
+  m.impl("longconv", &longconv_gpu);
   m.impl("filter_grad", &filter_grad_gpu);
 }
 
 TORCH_LIBRARY_IMPL(sffft, Autograd, m) {
+  m.impl("corr", &corr_autograd);
+  m.impl("longconv", &longconv_autograd);
   m.impl("spectrum", &spectrum_autograd);
   m.impl("conv", &conv_autograd);
 }

@@ -20,13 +20,11 @@ Gradients:
 
 - ``conv`` is differentiable in u. Causal convolution's adjoint is the anti-causal correlation
   du[m] = sum_{n >= m} dy[n] k[n - m]. With the N = 2L zero padding this is
-  IDFT(DFT(dy) * conj(K))[m] for m < L, so the backward pass runs the same kernel on the
-  conjugated spectrum (elementwise conjugation of the kernel-order buffer), with no time
-  reversal.
-- ``LongConv`` is differentiable in u and in the filter k. The filter gradient is the
-  batch-summed correlation dk[h, j] = sum_b sum_{n >= j} dy[b, h, n] u[b, h, n - j]: per
-  sequence the same correlation with u in the filter's place (``filter_grad``). The B*H input
-  rows become conjugated spectra of a batch-of-one convolution of the output gradients.
+  IDFT(DFT(dy) * conj(K))[m] for m < L, which ``torch.ops.sffft.corr(dy, kf, plan)`` computes from
+  conv's own spectrum: the same kernels with conjugate DFT and twiddle tables.
+- ``LongConv`` is differentiable in u and in the filter k (``torch.ops.sffft.longconv``). The filter
+  gradient is the batch-summed correlation dk[h, j] = sum_b sum_{n >= j} dy[b, h, n] u[b, h, n - j]
+  (``torch.ops.sffft.filter_grad``).
 - ``spectrum`` itself has no gradient and raises if its filter requires grad.
 """
 from __future__ import annotations
@@ -68,6 +66,16 @@ def _conv_fake(u, kf, plan):
     return torch.empty_like(u)
 
 
+@torch.library.register_fake("sffft::corr")
+def _corr_fake(u, kf, plan):
+    return _conv_fake(u, kf, plan)
+
+
+@torch.library.register_fake("sffft::longconv")
+def _longconv_fake(u, k, kf, plan):
+    return _conv_fake(u, kf, plan)
+
+
 @torch.library.register_fake("sffft::filter_grad")
 def _filter_grad_fake(u, dy):
     torch._check(u.dim() == 3 and dy.shape == u.shape, lambda: "u and dy must be [B, H, L]")
@@ -106,7 +114,8 @@ def filter_grad(u: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
 
 
 class _LongConvFn(torch.autograd.Function):
-    """y = conv(u, kf) with gradients for u and for the filter k that kf was made from."""
+    """y = conv(u, kf) with gradients for u and for the filter k that kf was made from, for the
+    multi-pass lengths (``torch.ops.sffft.longconv`` up to L = 16384)."""
 
     @staticmethod
     def forward(ctx, u, k, kf, fields):
@@ -119,7 +128,7 @@ class _LongConvFn(torch.autograd.Function):
         u, kf = ctx.saved_tensors
         du = dk = None
         if ctx.needs_input_grad[0]:
-            du = torch.ops.sffft.conv(dy.to(u.dtype).contiguous(), torch.conj_physical(kf), ctx.fields)
+            du = torch.ops.sffft.corr(dy.to(u.dtype).contiguous(), kf, ctx.fields)
         if ctx.needs_input_grad[1]:
             dk = filter_grad(u, dy)
         return du, dk, None, None
@@ -190,5 +199,7 @@ class LongConv:
         plan, fields = self._plan_and_fields(u)
         kf = self.spectrum(k, plan)
         if k.requires_grad and torch.is_grad_enabled():
+            if u.shape[-1] in LENGTHS:
+                return torch.ops.sffft.longconv(u, k, kf, fields)
             return _LongConvFn.apply(u, k, kf, fields)
         return torch.ops.sffft.conv(u, kf, fields)
