@@ -76,3 +76,17 @@ def test_legacy_and_fp16_accumulation(dev, L):
                     err = oracle.rel_l2(_run(dev, u, k, p, io), ref)
                     print(f"  rel_l2={err:.3e}", flush=True)
                     assert np.isfinite(err) and err <= bound(io, acc, p.seqs), (L, repr(p), io, err)
+
+
+@pytest.mark.parametrize("io", ["fp32", "bf16"])
+@pytest.mark.parametrize("L,spec", [(4096, "32x16x16"), (8192, "32x32x16")])
+def test_one_sequence_results_do_not_depend_on_the_wavefronts(dev, L, spec, io):
+    """The odd-batch plans' wavefront count is a matter of speed only: bit-identical results."""
+    import torch
+
+    u, k = oracle.gen_inputs(3, 5, L, seed=L)
+    u, k = torch.from_numpy(u).to(dev), torch.from_numpy(k).to(dev)
+    if io == "bf16":
+        u = sf.to_bf16(u)
+    y = [sf.conv(u, sf.spectrum(k, L, p), p) for p in (sf.make_plan(spec, 4), sf.make_plan(spec, 8))]
+    assert torch.equal(*y)
