@@ -575,7 +575,7 @@ SpectrumOrder spectrum_order(const sffft_plan* p, int whole, int conj) {
 // i ki for a complex filter (ki non-null, whole spectrum); with conj, its conjugate (the
 // spectrum the correlations of the backward passes run on). Zero-padded rows of up to 16384
 // points take one launch (spectrum.hpp), which leaves `work` alone: the three launches below took
-// 36.9, 122 and 188 us where it takes 10.8, 30 and 65 (H = 768, L = 1024, 4096, 8192), with the
+// 36.9, 121 and 184 us where it takes 9.6, 27.6 and 55 (H = 768, L = 1024, 4096, 8192), with the
 // same bits. Longer rows do not fit a workgroup's LDS; they, and the unpadded ones of a circular
 // convolution, are padded into `work` (H * N complex64), transformed there in place (fp64
 // stages, complex64 between them) and gathered into kernel order. Above 16384 points that is the two-pass transform, whose workspace is this call's own rows

@@ -24,7 +24,7 @@
 // moved 8 bytes a sample 11 times each way. Two wavefronts per SIMD (the fp64 planes take the
 // LDS) leave it bound by the latency between the barriers of the stages, so every launch requests
 // its points before it evaluates its tables. Measured at B=8, H=16, 256 x 256: 269 us in 13
-// launches -> 78 us, of which rows_forward 26, cols 25 + 5, rows_inverse 23 (2.6 to 3 TB/s each).
+// launches -> 72 us.
 #pragma once
 #include "transforms.hpp"
 
@@ -33,37 +33,6 @@ namespace xf {
 namespace c2 {
 
 constexpr int CB = 8;  // columns per block
-
-// The DFT of a line's R points in registers, natural order in, bit-reversed order out: line_dft with its
-// roots as constants (quarter turns cost nothing), conjugated with INV.
-template <int R, bool INV>
-__device__ __forceinline__ void line(double (&vr)[R], double (&vi)[R]) {
-  constexpr double c[5] = {1.0, 0.92387953251128675613, 0.70710678118654752440, 0.38268343236508977173, 0.0};
-#pragma unroll
-  for (int m = R; m >= 2; m >>= 1) {
-    const int h = m >> 1, step = 16 / m;
-#pragma unroll
-    for (int b = 0; b < R; b += m)
-#pragma unroll
-      for (int j = 0; j < h; j++) {
-        const int i0 = b + j, i1 = i0 + h, t = j * step;  // times exp(-2 pi i t / 16), t < 8
-        const double dr = vr[i0] - vr[i1], di = vi[i0] - vi[i1];
-        vr[i0] += vr[i1];
-        vi[i0] += vi[i1];
-        const double wr = t <= 4 ? c[t] : -c[8 - t], ws = t <= 4 ? c[4 - t] : c[t - 4], wi = INV ? ws : -ws;
-        if (t == 0) {
-          vr[i1] = dr;
-          vi[i1] = di;
-        } else if (t == 4) {
-          vr[i1] = INV ? -di : di;
-          vi[i1] = INV ? dr : -dr;
-        } else {
-          vr[i1] = dr * wr - di * wi;
-          vi[i1] = dr * wi + di * wr;
-        }
-      }
-  }
-}
 
 // What others read next has been written. The memory clobber keeps LDS reads above the barrier:
 // the compiler's sinking of instructions to their use does not take s_barrier for a store.
@@ -113,7 +82,7 @@ __device__ __forceinline__ void twiddled_line(Planes<G>& sh, int seq, int l, Loa
   double vr[R], vi[R];
 #pragma unroll
   for (int t = 0; t < R; t++) load(base + t * sJ, vr[t], vi[t]);
-  line<R, INV>(vr, vi);
+  line_dft<R>(vr, vi, INV ? 1 : -1);
   const int e = inner * (G::N / REST) * G::TSTEP;
   const double w1c = sh.tc[e], w1s = INV ? sh.ts[e] : -sh.ts[e];
   double wr = 1.0, wi = 0.0;
@@ -230,9 +199,9 @@ __global__ void __launch_bounds__(Rows<M>::THREADS)
   __shared__ Planes<G> sh;
   const int r0 = blockIdx.x * G::NSEQ;
   float2 x[MAX_RADIX];
-  load_first<G>(x, [&](int seq, int p) {
-    const int row = r0 + seq;
-    return row < nrows ? (row < nu ? u + (size_t)row * M : k + (size_t)(row - nu) * M)[p] : make_float2(0.f, 0.f);
+  load_first<G>(x, [&](int seq, int p) {  // lanes past the last row repeat it
+    const int row = r0 + seq < nrows ? r0 + seq : nrows - 1;
+    return (row < nu ? u + (size_t)row * M : k + (size_t)(row - nu) * M)[p];
   });
   sh.init();
   __syncthreads();
@@ -248,7 +217,7 @@ __global__ void __launch_bounds__(Rows<M>::THREADS)
       vr[t] = sh.re[at];
       vi[t] = sh.im[at];
     }
-    line<R, false>(vr, vi);
+    line_dft<R>(vr, vi, -1);
 #pragma unroll
     for (int t = 0; t < R; t++) sh.put(G::at(seq, l * R + t), vr[bitrev<R>(t)], vi[bitrev<R>(t)]);
   }
@@ -281,11 +250,9 @@ __global__ void __launch_bounds__(Rows<M>::THREADS)
 #pragma unroll
   for (int v = 0; v < G::SLOTS / 2 / G::THREADS; v++) {
     const int i = threadIdx.x + v * G::THREADS, g = (i / CB) % G::NSEQ, f = i / (CB * G::NSEQ) * CB + i % CB;
-    xa[v] = xz[v] = make_float2(0.f, 0.f);
-    if (r0 + g < nrows) {
-      xa[v] = spec[spec_at(r0 + g, f, l0, M)];
-      xz[v] = spec[spec_at(r0 + g, f ? M - f : M / 2, l0, M)];
-    }
+    const int row = r0 + g < nrows ? r0 + g : nrows - 1;  // lanes past the last row repeat it
+    xa[v] = spec[spec_at(row, f, l0, M)];
+    xz[v] = spec[spec_at(row, f ? M - f : M / 2, l0, M)];
   }
   __asm__ volatile("" ::: "memory");
   sh.init();
@@ -323,7 +290,7 @@ __global__ void __launch_bounds__(Rows<M>::THREADS)
       vr[t] = sh.re[at];
       vi[t] = sh.im[at];
     }
-    line<R, true>(vr, vi);
+    line_dft<R>(vr, vi, 1);
     if (r0 + seq >= nrows) continue;
     float2* o = y + (size_t)(r0 + seq) * M + kb;
 #pragma unroll
@@ -376,7 +343,7 @@ __device__ __forceinline__ void cols_back(ColsShared<N0, true>& sh, Dst dst) {
       wi = fma(wr, w1s, wi * w1c);
       wr = nr;
     }
-    line<R, true>(vr, vi);
+    line_dft<R>(vr, vi, 1);
 #pragma unroll
     for (int t = 0; t < R; t++) {
       if constexpr (REST == N0) dst(seq, base + t * sJ, vr[bitrev<R>(t)], vi[bitrev<R>(t)]);
@@ -403,7 +370,8 @@ __global__ void __launch_bounds__(Cols<N0>::THREADS)
   auto live = [&](int seq) { return b0 + seq / CB < nblocks; };
   float2 x0[MAX_RADIX];
   load_first<G>(x0, [&](int seq, int p) {
-    return live(seq) ? x[seq / CB * G::BLOCK + p * CB + seq % CB] : make_float2(0.f, 0.f);
+    const int blk = live(seq) ? seq / CB : nblocks - 1 - b0;  // lanes past the last block repeat it
+    return x[blk * G::BLOCK + p * CB + seq % CB];
   });
   sh.s.init();
   __syncthreads();
@@ -434,7 +402,7 @@ __global__ void __launch_bounds__(Cols<N0>::THREADS)
       ar[t] = sh.s.re[at];
       ai[t] = sh.s.im[at];
     }
-    line<R, false>(ar, ai);
+    line_dft<R>(ar, ai, -1);
 #pragma unroll
     for (int t = 0; t < R; t++) {
       vr[m][t] = ar[bitrev<R>(t)];
@@ -480,7 +448,7 @@ __global__ void __launch_bounds__(Cols<N0>::THREADS)
           ai[t] = Pi + Qr;
         }
       }
-      line<R, true>(ar, ai);
+      line_dft<R>(ar, ai, 1);
 #pragma unroll
       for (int t = 0; t < R; t++) {
         if constexpr (N0 > MAX_RADIX) {

@@ -63,50 +63,40 @@ __host__ __device__ inline SpectrumPair spectrum_pair(const SpectrumOrder& o, in
 // line_dft whose first radix-2 level has nothing to add, and for a real row no imaginary part. The
 // rounding steps that remain are line_dft's.
 template <bool CPLX>
-__device__ __forceinline__ void padded_line_dft(double (&vr)[16], double (&vi)[16], const double* wc,
-                                                const double* ws) {
+__device__ __forceinline__ void padded_line_dft(double (&vr)[16], double (&vi)[16]) {
 #pragma clang fp contract(off)
+  constexpr double c16[5] = {1.0, 0.92387953251128675613, 0.70710678118654752440, 0.38268343236508977173, 0.0};
+  double ar[2][8], ai[2][8];
 #pragma unroll
   for (int j = 0; j < 8; j++) {
-    const double ar = vr[j], ai = CPLX ? vi[j] : 0.0;
+    const double xr = vr[j], xi = CPLX ? vi[j] : 0.0;
+    const double c = j <= 4 ? c16[j] : -c16[8 - j], sn = -(j <= 4 ? c16[4 - j] : c16[j - 4]);
+    ar[0][j] = xr;
+    ai[0][j] = xi;
     if (j == 0) {
-      vr[8] = ar;
-      vi[8] = ai;
+      ar[1][j] = xr;
+      ai[1][j] = xi;
+    } else if (j == 4) {
+      ar[1][j] = xi;
+      ai[1][j] = -xr;
     } else if (CPLX) {
-      vr[j + 8] = fma(ar, wc[j], -(ai * ws[j]));
-      vi[j + 8] = fma(ar, ws[j], ai * wc[j]);
+      ar[1][j] = fma(xr, c, -(xi * sn));
+      ai[1][j] = fma(xr, sn, xi * c);
     } else {
-      vr[j + 8] = ar * wc[j];
-      vi[j + 8] = ar * ws[j];
+      ar[1][j] = xr * c;
+      ai[1][j] = xr * sn;
     }
-    if (!CPLX) vi[j] = 0.0;
   }
-  // the two halves: 8-point transforms, their roots every second one of the table
-  auto half8 = [&](int o) {
+  // the remaining levels: two 8-point transforms, each in bit-reversed order
 #pragma unroll
-    for (int m = 8; m >= 2; m >>= 1) {
-      const int h = m >> 1, step = 16 / m;
+  for (int o = 0; o < 2; o++) {
+    xf::line_dft<8>(ar[o], ai[o], -1);
 #pragma unroll
-      for (int b = 0; b < 8; b += m)
-#pragma unroll
-        for (int j = 0; j < h; j++) {
-          const int i0 = o + b + j, i1 = i0 + h;
-          const double ar = vr[i0], ai = vi[i0], dr = ar - vr[i1], di = ai - vi[i1];
-          vr[i0] = ar + vr[i1];
-          vi[i0] = ai + vi[i1];
-          if (j == 0) {
-            vr[i1] = dr;
-            vi[i1] = di;
-          } else {
-            const double c = wc[j * step], sn = ws[j * step];
-            vr[i1] = fma(dr, c, -(di * sn));
-            vi[i1] = fma(dr, sn, di * c);
-          }
-        }
+    for (int j = 0; j < 8; j++) {
+      vr[8 * o + j] = ar[o][j];
+      vi[8 * o + j] = ai[o][j];
     }
-  };
-  half8(0);
-  half8(8);
+  }
 }
 
 // Lanes: one radix-16 line each, at least a wavefront.
@@ -124,26 +114,17 @@ __global__ void __launch_bounds__(SpectrumGeom<N>::THREADS)
   constexpr int R = xf::MAX_RADIX, sJ = N / R, L = N / 2;
   static_assert(R == 16 && N >= 32, "the first stage is a padded radix-16 line");
   __shared__ float2 buf[SG::SLOTS + SG::SLOTS / 16];
-  __shared__ double wc[R], ws[R];
   __shared__ double tc[sJ], ts[sJ];
   const int g = threadIdx.x / sJ, inner = threadIdx.x % sJ, h0 = blockIdx.x * SG::G;
+  // in flight while the table is evaluated; lanes past the last row repeat it
   float xr[8], xi[8];
+  const size_t first = (size_t)(h0 + g < H ? h0 + g : H - 1) * L + inner;
 #pragma unroll
-  for (int t = 0; t < 8; t++) xr[t] = xi[t] = 0.f;
-  if (h0 + g < H) {
-    const size_t row = (size_t)(h0 + g) * L + inner;
-#pragma unroll
-    for (int t = 0; t < 8; t++) {
-      xr[t] = kr[row + t * sJ];
-      if (CPLX) xi[t] = ki[row + t * sJ];
-    }
+  for (int t = 0; t < 8; t++) {
+    xr[t] = kr[first + t * sJ];
+    xi[t] = CPLX ? ki[first + t * sJ] : 0.f;
   }
-  if (threadIdx.x < R) {
-    double sn, c;
-    sincospi(2.0 * (double)threadIdx.x / (double)R, &sn, &c);
-    wc[threadIdx.x] = c;
-    ws[threadIdx.x] = -sn;
-  }
+  __asm__ volatile("" ::: "memory");
   // one sincospi per entry of the twiddle bases, as line_kernel evaluates them
   if (threadIdx.x < sJ) {
     double sn, c;
@@ -159,12 +140,12 @@ __global__ void __launch_bounds__(SpectrumGeom<N>::THREADS)
       vr[t] = (double)xr[t];
       vi[t] = (double)xi[t];
     }
-    padded_line_dft<CPLX>(vr, vi, wc, ws);
+    padded_line_dft<CPLX>(vr, vi);
     xf::twiddled_outputs_w<R>(vr, vi, tc[inner], -ts[inner],
                               [&](int k, float2 v) { buf[xf::lpad(g * N + inner + k * sJ)] = v; });
   }
   __syncthreads();
-  xf::line_stage<N, N / R, SG::G, SG::THREADS>(buf, wc, ws, tc, ts, -1, 1.f);
+  xf::line_stage<N, N / R, SG::G, SG::THREADS>(buf, tc, ts, -1, 1.f);
   for (int i = threadIdx.x; i < SG::SLOTS / 2; i += SG::THREADS) {
     const int row = i / L, f = i - row * L;
     if (h0 + row >= H) break;

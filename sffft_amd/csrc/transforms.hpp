@@ -23,10 +23,7 @@
 namespace sffft {
 namespace xf {
 
-#ifndef SFFFT_XF_MAX_RADIX
-#define SFFFT_XF_MAX_RADIX 16
-#endif
-constexpr int MAX_RADIX = SFFFT_XF_MAX_RADIX;
+constexpr int MAX_RADIX = 16;
 constexpr int MAX_STAGES = 6;
 constexpr long long MAX_N = 1LL << 24;
 constexpr long long MAX_ELEMS = 1LL << 31;  // sequences * N per call
@@ -71,31 +68,43 @@ struct Seqs {
   }
 };
 
-// The radix-R DFT of one line's R points, in registers, shared by both kernels below:
+// x with its sign flipped where neg (0 or INT_MIN) says so
+__device__ __forceinline__ double flip(double x, int neg) {
+  return __hiloint2double(__double2hiint(x) ^ neg, __double2loint(x));
+}
+
+// The radix-R DFT of one line's R points, in registers, shared by all kernels below:
 // radix-2 decimation in frequency over log2(R) levels, natural input order, bit-reversed
-// output order, in fp64 with w_m^j = w_T^(j * T / m) read from a table of the T-th roots
-// of unity. About R*log2(R)/2 complex products instead of the R*R of the dense sum.
-// Contraction is off and the complex products are written with fma, so every kernel
-// that inlines this rounds in the same places and gets the same bits.
-template <int R, int T>
-__device__ __forceinline__ void line_dft(double (&vr)[R], double (&vi)[R], const double* wc, const double* ws) {
+// output order, in fp64, exponents of the given sign. The 16th roots of unity are constants
+// (scalar registers; from an LDS table they took 32 VGPRs and the reads), the sign goes into their
+// sines on the scalar unit, and the quarter turn is a swap. About R*log2(R)/2 complex products
+// instead of the R*R of the dense sum. Contraction is off and the complex products are written
+// with fma, so every kernel that inlines this rounds in the same places and gets the same bits.
+template <int R>
+__device__ __forceinline__ void line_dft(double (&vr)[R], double (&vi)[R], int sign) {
 #pragma clang fp contract(off)
+  static_assert(R <= 16, "16th roots");
+  constexpr double c16[5] = {1.0, 0.92387953251128675613, 0.70710678118654752440, 0.38268343236508977173, 0.0};
+  const int neg = sign < 0 ? (int)0x80000000 : 0;
 #pragma unroll
   for (int m = R; m >= 2; m >>= 1) {
-    const int h = m >> 1, step = T / m;
+    const int h = m >> 1, step = 16 / m;
 #pragma unroll
     for (int b = 0; b < R; b += m)
 #pragma unroll
       for (int j = 0; j < h; j++) {
-        const int i0 = b + j, i1 = i0 + h;
+        const int i0 = b + j, i1 = i0 + h, t = j * step;  // times w_16^t, t < 8
         const double ar = vr[i0], ai = vi[i0], dr = ar - vr[i1], di = ai - vi[i1];
         vr[i0] = ar + vr[i1];
         vi[i0] = ai + vi[i1];
-        if (j == 0) {
+        if (t == 0) {
           vr[i1] = dr;
           vi[i1] = di;
+        } else if (t == 4) {
+          vr[i1] = flip(-di, neg);
+          vi[i1] = flip(dr, neg);
         } else {
-          const double c = wc[j * step], sn = ws[j * step];
+          const double c = t < 4 ? c16[t] : -c16[8 - t], sn = flip(t < 4 ? c16[4 - t] : c16[t - 4], neg);
           vr[i1] = fma(dr, c, -(di * sn));
           vi[i1] = fma(dr, sn, di * c);
         }
@@ -142,14 +151,6 @@ template <int R>
 __global__ void __launch_bounds__(128)
     stage_kernel(const float2* in, float2* out, float2* work, Seqs q, Radices d, int J, int N, int sign,
                  float scale) {
-  __shared__ double wc[R], ws[R];
-  for (int i = threadIdx.x; i < R; i += blockDim.x) {
-    double sn, c;
-    sincospi(2.0 * (double)i / (double)R, &sn, &c);
-    wc[i] = c;
-    ws[i] = sign * sn;  // w_R^i = c + i * ws[i]
-  }
-  __syncthreads();
   const int S = d.S;
   int sJ = 1;
   for (int i = J + 1; i < S; i++) sJ *= d.r[i];
@@ -191,7 +192,7 @@ __global__ void __launch_bounds__(128)
     vr[t] = (double)x[t].x;
     vi[t] = (double)x[t].y;
   }
-  line_dft<R, R>(vr, vi, wc, ws);
+  line_dft<R>(vr, vi, sign);
   if (last) {
 #pragma unroll
     for (int k = 0; k < R; k++) {
@@ -217,6 +218,9 @@ constexpr int ONEPASS_MAX_N = 16384;  // 136 KB of LDS
 constexpr int ONEPASS_SLOTS = 4096;
 
 __device__ __forceinline__ int lpad(int p) { return p + (p >> 4); }
+// with EXTRA, one more slot per EXTRA elements
+template <int EXTRA>
+__device__ __forceinline__ int lpadx(int p) { return lpad(p) + (EXTRA ? p / (EXTRA ? EXTRA : 1) : 0); }
 
 template <int N>
 struct LineGeom {
@@ -224,50 +228,86 @@ struct LineGeom {
   static constexpr int SLOTS = G * N;
   // one thread per radix-16 line: 256 threads, 512 at N = 8192, 1024 at N = 16384
   static constexpr int THREADS = SLOTS / MAX_RADIX;
-  static constexpr int LDS = SLOTS + SLOTS / 16;
+  // The last stage takes its lines in the order of their frequencies, so that its stores are
+  // contiguous; those lines start N / 16 elements apart, which a slot of padding each spreads over
+  // the banks (N >= 4096: the shorter strides already fall on several).
+  static constexpr int EXTRA = N >= 4096 ? N / 16 : 0;
+  static constexpr int LDS = SLOTS + SLOTS / 16 + (EXTRA ? 16 : 0);
+  // From N = 256 the first stage loads runs of 128 bytes and more straight into registers.
+  static constexpr bool DIRECT = N >= 256;
   // twiddle bases of the non-last stages: w_N^j for j < N / 16 (w_Nj^inner = w_N^(inner N/Nj))
   static constexpr int TW = N / MAX_RADIX > 1 ? N / MAX_RADIX : 1;
   // radix of the stage whose remaining product of radices is REST (16s first)
   static constexpr int radix(int rest) { return rest > MAX_RADIX ? MAX_RADIX : rest; }
+  static constexpr int last() {  // of the last stage
+    int r = N;
+    while (r > MAX_RADIX) r /= MAX_RADIX;
+    return r;
+  }
 };
 
-// One stage over the workgroup's lines: REST is the product of this and the later
-// radices (REST = N at the first stage), R this stage's radix, sJ = REST / R its stride.
+// Orders the workgroup's LDS accesses; global accesses stay in flight.
+// The memory clobbers keep LDS reads above the barrier: the compiler's sinking of instructions to
+// their use does not take s_barrier for a store.
+__device__ __forceinline__ void lds_sync() {
+  __asm__ volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  __asm__ volatile("" ::: "memory");
+}
+
+// The stages before the last one, from the one whose remaining product of radices is REST (REST =
+// N at the first stage): R = 16, sJ = REST / R its stride, each followed by a barrier.
 // tc, ts: the workgroup's table of w_N^j = tc[j] + i sign ts[j], j < N/16. A line's twiddle
 // base w_REST^inner is entry inner * N/REST: sincospi of 2j/N there and of 2 inner/REST in
 // the staged kernel are the same exact fp64 argument, so both paths get the same bits.
 // G sequences of N in buf, THREADS threads (the one-pass kernel's geometry by default).
-template <int N, int REST, int G = LineGeom<N>::G, int THREADS = LineGeom<N>::THREADS>
-__device__ __forceinline__ void line_stage(float2* buf, const double* wc, const double* ws, const double* tc,
-                                           const double* ts, int sign, float scale) {
+template <int N, int REST, int G = LineGeom<N>::G, int THREADS = LineGeom<N>::THREADS, int EXTRA = 0>
+__device__ __forceinline__ void line_stages(float2* buf, const double* tc, const double* ts, int sign) {
   constexpr int R = LineGeom<N>::radix(REST), sJ = REST / R, LPS = N / R;
-  constexpr int LINES = G * LPS;
-  constexpr bool LAST = REST == R;
-  for (int li = threadIdx.x; li < LINES; li += THREADS) {
-    const int g = li / LPS, l = li - g * LPS;
-    const int inner = l % sJ, base = g * N + (l / sJ) * REST + inner;
+  if constexpr (sJ > 1) {
+    for (int li = threadIdx.x; li < G * LPS; li += THREADS) {
+      const int g = li / LPS, l = li - g * LPS;
+      const int inner = l % sJ, base = g * N + (l / sJ) * REST + inner;
+      double vr[R], vi[R];
+#pragma unroll
+      for (int t = 0; t < R; t++) {
+        const float2 x = buf[lpadx<EXTRA>(base + t * sJ)];
+        vr[t] = (double)x.x;
+        vi[t] = (double)x.y;
+      }
+      line_dft<R>(vr, vi, sign);
+      const int j = inner * (N / REST);
+      twiddled_outputs_w<R>(vr, vi, tc[j], sign * ts[j],
+                            [&](int k, float2 v) { buf[lpadx<EXTRA>(base + k * sJ)] = v; });
+    }
+    lds_sync();
+    line_stages<N, REST / R, G, THREADS, EXTRA>(buf, tc, ts, sign);
+  }
+}
+
+// All stages from REST on, the last one in place too, scaled: element base + k of a line holds its
+// frequency digit k.
+template <int N, int REST, int G = LineGeom<N>::G, int THREADS = LineGeom<N>::THREADS>
+__device__ __forceinline__ void line_stage(float2* buf, const double* tc, const double* ts, int sign, float scale) {
+  line_stages<N, REST, G, THREADS>(buf, tc, ts, sign);
+  constexpr int R = LineGeom<N>::last(), LPS = N / R;
+  for (int li = threadIdx.x; li < G * LPS; li += THREADS) {
     double vr[R], vi[R];
 #pragma unroll
     for (int t = 0; t < R; t++) {
-      const float2 x = buf[lpad(base + t * sJ)];
+      const float2 x = buf[lpad(li * R + t)];
       vr[t] = (double)x.x;
       vi[t] = (double)x.y;
     }
-    line_dft<R, MAX_RADIX>(vr, vi, wc, ws);
-    if constexpr (LAST) {
-      // in place, scaled: element base + k holds frequency digit k of this line
+    line_dft<R>(vr, vi, sign);
 #pragma unroll
-      for (int k = 0; k < R; k++) {
-        const int r = bitrev<R>(k);
-        buf[lpad(base + k)] = make_float2((float)(vr[r] * scale), (float)(vi[r] * scale));
-      }
-    } else {
-      const int j = inner * (N / REST);
-      twiddled_outputs_w<R>(vr, vi, tc[j], sign * ts[j], [&](int k, float2 v) { buf[lpad(base + k * sJ)] = v; });
+    for (int k = 0; k < R; k++) {
+      const int r = bitrev<R>(k);
+      buf[lpad(li * R + k)] = make_float2((float)(vr[r] * scale), (float)(vi[r] * scale));
     }
   }
-  __syncthreads();
-  if constexpr (!LAST) line_stage<N, REST / R, G, THREADS>(buf, wc, ws, tc, ts, sign, scale);
+  lds_sync();
 }
 
 // Position in the line, after the last stage, of natural-order frequency f: the digits
@@ -288,18 +328,32 @@ __device__ __forceinline__ int line_position(int f) {
   return base + f / W;
 }
 
+// Measured (768 x 16384, 1536 x 8192, 6144 x 2048, 49152 x 256): with the sequence staged through LDS
+// on the way in and out and the roots of unity in LDS 97.5, 93, 83 and 71 us; this 62, 53.5, 46 and
+// 44.5 (3.2 to 4.5 TB/s; a copy 5.2). At N >= 8192 one or two workgroups fill a CU and the
+// round trips to memory at either end of a sequence show. Workgroups that stay and request the next
+// sequence while they transform one spill (18 to 22 VGPRs at 128) and took 76 and 77 us.
 template <int N>
 __global__ void __launch_bounds__(LineGeom<N>::THREADS)
     line_kernel(const float2* in, float2* out, Seqs q, int sign, float scale) {
   typedef LineGeom<N> LG;
   __shared__ float2 buf[LG::LDS];
-  __shared__ double wc[MAX_RADIX], ws[MAX_RADIX];
   __shared__ double tc[LG::TW], ts[LG::TW];
-  if (threadIdx.x < MAX_RADIX) {
-    double sn, c;
-    sincospi(2.0 * (double)threadIdx.x / (double)MAX_RADIX, &sn, &c);
-    wc[threadIdx.x] = c;
-    ws[threadIdx.x] = sign * sn;
+  constexpr int R = LG::last(), LPS = N / R;
+  const long long s0 = (long long)blockIdx.x * LG::G;
+  const int G = q.nseq - s0 < LG::G ? (int)(q.nseq - s0) : LG::G;
+  // the first stage's line of this lane: points inner + sJ t of sequence s0 + gt, in flight while
+  // the tables are evaluated
+  constexpr int sJ = LG::DIRECT ? N / MAX_RADIX : 1;
+  const int gt = threadIdx.x / sJ, inner = threadIdx.x % sJ;
+  float2 x[MAX_RADIX];
+  if constexpr (LG::DIRECT) {
+    // lanes past the last sequence repeat it and store nothing: a zero instead of the load, chosen
+    // per point, became a branch and a wait per point
+    const float2* src = in + q.base(s0 + (gt < G ? gt : G - 1)) + inner;
+#pragma unroll
+    for (int t = 0; t < MAX_RADIX; t++) x[t] = src[t * sJ];
+    __asm__ volatile("" ::: "memory");
   }
   // one sincospi per table entry instead of one per line and stage
   for (int j = threadIdx.x; j < LG::TW; j += LG::THREADS) {
@@ -308,17 +362,47 @@ __global__ void __launch_bounds__(LineGeom<N>::THREADS)
     tc[j] = c;
     ts[j] = sn;
   }
-  const long long s0 = (long long)blockIdx.x * LG::G;
-  const int G = q.nseq - s0 < LG::G ? (int)(q.nseq - s0) : LG::G;
-  for (int i = threadIdx.x; i < LG::SLOTS; i += LG::THREADS) {
-    const int g = i / N;
-    buf[lpad(i)] = g < G ? in[q.base(s0 + g) + (i - g * N)] : make_float2(0.f, 0.f);
+  if constexpr (LG::DIRECT) {
+    lds_sync();
+    double vr[MAX_RADIX], vi[MAX_RADIX];
+#pragma unroll
+    for (int t = 0; t < MAX_RADIX; t++) {
+      vr[t] = (double)x[t].x;
+      vi[t] = (double)x[t].y;
+    }
+    line_dft<MAX_RADIX>(vr, vi, sign);
+    twiddled_outputs_w<MAX_RADIX>(vr, vi, tc[inner], sign * ts[inner], [&](int k, float2 v) {
+      buf[lpadx<LG::EXTRA>(gt * N + inner + k * sJ)] = v;
+    });
+    lds_sync();
+    line_stages<N, N / MAX_RADIX, LG::G, LG::THREADS, LG::EXTRA>(buf, tc, ts, sign);
+  } else {
+    for (int i = threadIdx.x; i < LG::SLOTS; i += LG::THREADS) {
+      const int g = i / N;
+      buf[lpad(i)] = g < G ? in[q.base(s0 + g) + (i - g * N)] : make_float2(0.f, 0.f);
+    }
+    __syncthreads();
+    line_stages<N, N>(buf, tc, ts, sign);
   }
-  __syncthreads();
-  line_stage<N, N>(buf, wc, ws, tc, ts, sign, scale);
-  for (int i = threadIdx.x; i < G * N; i += LG::THREADS) {
-    const int g = i / N, f = i - g * N;
-    out[q.base(s0 + g) + f] = buf[lpad(g * N + line_position<N>(f))];
+  // last stage, to memory: line kb of a sequence holds its frequencies kb + LPS k
+  for (int li = threadIdx.x; li < LG::G * LPS; li += LG::THREADS) {
+    const int g = li / LPS, kb = li - g * LPS, at = g * N + line_position<N>(kb);
+    double vr[R], vi[R];
+#pragma unroll
+    for (int t = 0; t < R; t++) {
+      const float2 v = buf[lpadx<LG::EXTRA>(at + t)];
+      vr[t] = (double)v.x;
+      vi[t] = (double)v.y;
+    }
+    line_dft<R>(vr, vi, sign);
+    if (g < G) {
+      float2* dst = out + q.base(s0 + g) + kb;
+#pragma unroll
+      for (int k = 0; k < R; k++) {
+        const int r = bitrev<R>(k);
+        dst[k * LPS] = make_float2((float)(vr[r] * scale), (float)(vi[r] * scale));
+      }
+    }
   }
 }
 
@@ -379,58 +463,48 @@ struct RowGeom {
   static constexpr int LDS = SLOTS + SLOTS / 16;
 };
 
-// stage of pass A whose local stride is LS (N1/16 at the first stage, 1 at the last)
+// Stage of pass A whose local stride is LS (N1/16 at the first stage, 1 at the last), one line per
+// lane: the first one from `src`, the last one to `dst` (columns c0.., N2 points from row to row: runs of
+// C points either way), through buf between them.
 template <int N1, int LS>
-__device__ __forceinline__ void col_stage(float2* buf, const double* wc, const double* ws, int c0, int N2,
-                                          int sign) {
-  constexpr int R = MAX_RADIX, C = ColGeom<N1>::C, LINES = (N1 / R) * C;
-  for (int li = threadIdx.x; li < LINES; li += ColGeom<N1>::THREADS) {
-    const int j = li % C, l = li / C;  // column j (consecutive across threads), line l of it
-    const int lu = l % LS, mb = (l / LS) * R * LS + lu;
-    double vr[R], vi[R];
+__device__ __forceinline__ void col_stage(const float2* src, float2* dst, float2* buf, int c0, int N2, int sign) {
+  constexpr int R = MAX_RADIX, C = ColGeom<N1>::C;
+  static_assert((N1 / R) * C == ColGeom<N1>::THREADS, "a line per lane");
+  const int j = threadIdx.x % C, l = threadIdx.x / C;  // column j (consecutive across threads), line l of it
+  const int lu = l % LS, mb = (l / LS) * R * LS + lu;
+  float2 x[R];
 #pragma unroll
-    for (int t = 0; t < R; t++) {
-      const float2 x = buf[(mb + t * LS) * C + j];
-      vr[t] = (double)x.x;
-      vi[t] = (double)x.y;
-    }
-    line_dft<R, R>(vr, vi, wc, ws);
-    // the stage kernel's twiddle of this line: inner = p mod sJ, Nj = R sJ, sJ = LS N2
-    twiddled_outputs<R>(vr, vi, c0 + j + lu * N2, R * LS * N2, sign,
-                        [&](int k, float2 v) { buf[(mb + k * LS) * C + j] = v; });
+  for (int t = 0; t < R; t++) {
+    if constexpr (LS == N1 / R) x[t] = src[(long long)(mb + t * LS) * N2 + j];
+    else x[t] = buf[(mb + t * LS) * C + j];
   }
-  __syncthreads();
-  if constexpr (LS > 1) col_stage<N1, LS / R>(buf, wc, ws, c0, N2, sign);
+  double vr[R], vi[R];
+#pragma unroll
+  for (int t = 0; t < R; t++) {
+    vr[t] = (double)x[t].x;
+    vi[t] = (double)x[t].y;
+  }
+  line_dft<R>(vr, vi, sign);
+  // the stage kernel's twiddle of this line: inner = p mod sJ, Nj = R sJ, sJ = LS N2
+  twiddled_outputs<R>(vr, vi, c0 + j + lu * N2, R * LS * N2, sign, [&](int k, float2 v) {
+    if constexpr (LS == 1) dst[(long long)(mb + k) * N2 + j] = v;
+    else buf[(mb + k * LS) * C + j] = v;
+  });
+  if constexpr (LS > 1) {
+    lds_sync();
+    col_stage<N1, LS / R>(src, dst, buf, c0, N2, sign);
+  }
 }
 
 template <int N1>
 __global__ void __launch_bounds__(ColGeom<N1>::THREADS)
     col_kernel(const float2* in, float2* work, Seqs q, int N2, int sign) {
   typedef ColGeom<N1> CG;
-  __shared__ float2 buf[CG::SLOTS];
-  __shared__ double wc[MAX_RADIX], ws[MAX_RADIX];
-  if (threadIdx.x < MAX_RADIX) {
-    double sn, c;
-    sincospi(2.0 * (double)threadIdx.x / (double)MAX_RADIX, &sn, &c);
-    wc[threadIdx.x] = c;
-    ws[threadIdx.x] = sign * sn;
-  }
+  __shared__ float2 buf[N1 > MAX_RADIX ? CG::SLOTS : 1];
   const int per_seq = N2 / CG::C;
   const long long s = blockIdx.x / per_seq;
   const int c0 = (int)(blockIdx.x - s * per_seq) * CG::C;
-  const long long N = (long long)N1 * N2;
-  const float2* src = in + q.base(s) + c0;
-  for (int i = threadIdx.x; i < CG::SLOTS; i += CG::THREADS) {
-    const int m = i / CG::C, j = i - m * CG::C;
-    buf[i] = src[(long long)m * N2 + j];
-  }
-  __syncthreads();
-  col_stage<N1, N1 / MAX_RADIX>(buf, wc, ws, c0, N2, sign);
-  float2* dst = work + s * N + c0;
-  for (int i = threadIdx.x; i < CG::SLOTS; i += CG::THREADS) {
-    const int m = i / CG::C, j = i - m * CG::C;
-    dst[(long long)m * N2 + j] = buf[i];
-  }
+  col_stage<N1, N1 / MAX_RADIX>(in + q.base(s) + c0, work + s * N1 * N2 + c0, buf, c0, N2, sign);
 }
 
 // b's k base-16 digits reversed (an involution)
@@ -443,19 +517,29 @@ __device__ __forceinline__ int digit_reverse16(int b, int k) {
   return r;
 }
 
+// N2 >= 256: the first stage's lines straight from memory. The last stage's go straight to it, the
+// G frequencies of one index next to each other. Measured, both passes, staged through LDS at either
+// end and now: 96 x 131072 120 -> 85 us, 48 x 2^18 124 -> 98, 16 x 2^20 217 -> 185.
 template <int N2>
 __global__ void __launch_bounds__(RowGeom<N2>::THREADS)
     row_kernel(const float2* work, float2* out, Seqs q, int N1, int k, int sign, float scale) {
   typedef RowGeom<N2> RG;
   typedef LineGeom<N2> LG;
   __shared__ float2 buf[RG::LDS];
-  __shared__ double wc[MAX_RADIX], ws[MAX_RADIX];
   __shared__ double tc[LG::TW], ts[LG::TW];
-  if (threadIdx.x < MAX_RADIX) {
-    double sn, c;
-    sincospi(2.0 * (double)threadIdx.x / (double)MAX_RADIX, &sn, &c);
-    wc[threadIdx.x] = c;
-    ws[threadIdx.x] = sign * sn;
+  constexpr int R = LG::last(), LPS = N2 / R, sJ = LG::DIRECT ? N2 / MAX_RADIX : 1;
+  const int per_seq = N1 / RG::G;
+  const long long s = blockIdx.x / per_seq;
+  const int r0 = (int)(blockIdx.x - s * per_seq) * RG::G;  // rev(b) of the first block
+  const long long N = (long long)N1 * N2;
+  const float2* src = work + s * N;
+  const int gt = threadIdx.x / sJ, inner = threadIdx.x % sJ;
+  float2 x[MAX_RADIX];
+  if constexpr (LG::DIRECT) {
+    const float2* row = src + (long long)digit_reverse16(r0 + gt, k) * N2 + inner;
+#pragma unroll
+    for (int t = 0; t < MAX_RADIX; t++) x[t] = row[t * sJ];
+    __asm__ volatile("" ::: "memory");
   }
   for (int j = threadIdx.x; j < LG::TW; j += RG::THREADS) {
     double sn, c;
@@ -463,21 +547,43 @@ __global__ void __launch_bounds__(RowGeom<N2>::THREADS)
     tc[j] = c;
     ts[j] = sn;
   }
-  const int per_seq = N1 / RG::G;
-  const long long s = blockIdx.x / per_seq;
-  const int r0 = (int)(blockIdx.x - s * per_seq) * RG::G;  // rev(b) of the first block
-  const long long N = (long long)N1 * N2;
-  const float2* src = work + s * N;
-  for (int i = threadIdx.x; i < RG::SLOTS; i += RG::THREADS) {
-    const int g = i / N2, e = i - g * N2;
-    buf[lpad(i)] = src[(long long)digit_reverse16(r0 + g, k) * N2 + e];
+  if constexpr (LG::DIRECT) {
+    lds_sync();
+    double vr[MAX_RADIX], vi[MAX_RADIX];
+#pragma unroll
+    for (int t = 0; t < MAX_RADIX; t++) {
+      vr[t] = (double)x[t].x;
+      vi[t] = (double)x[t].y;
+    }
+    line_dft<MAX_RADIX>(vr, vi, sign);
+    twiddled_outputs_w<MAX_RADIX>(vr, vi, tc[inner], sign * ts[inner],
+                                  [&](int kk, float2 v) { buf[lpad(gt * N2 + inner + kk * sJ)] = v; });
+    lds_sync();
+    line_stages<N2, N2 / MAX_RADIX, RG::G, RG::THREADS>(buf, tc, ts, sign);
+  } else {
+    for (int i = threadIdx.x; i < RG::SLOTS; i += RG::THREADS) {
+      const int g = i / N2, e = i - g * N2;
+      buf[lpad(i)] = src[(long long)digit_reverse16(r0 + g, k) * N2 + e];
+    }
+    __syncthreads();
+    line_stages<N2, N2, RG::G, RG::THREADS>(buf, tc, ts, sign);
   }
-  __syncthreads();
-  line_stage<N2, N2, RG::G, RG::THREADS>(buf, wc, ws, tc, ts, sign, scale);
   float2* dst = out + q.base(s) + r0;
-  for (int i = threadIdx.x; i < RG::SLOTS; i += RG::THREADS) {
-    const int f = i / RG::G, g = i - f * RG::G;
-    dst[(long long)f * N1 + g] = buf[lpad(g * N2 + line_position<N2>(f))];
+  for (int li = threadIdx.x; li < RG::G * LPS; li += RG::THREADS) {
+    const int g = li % RG::G, kb = li / RG::G, at = g * N2 + line_position<N2>(kb);
+    double vr[R], vi[R];
+#pragma unroll
+    for (int t = 0; t < R; t++) {
+      const float2 v = buf[lpad(at + t)];
+      vr[t] = (double)v.x;
+      vi[t] = (double)v.y;
+    }
+    line_dft<R>(vr, vi, sign);
+#pragma unroll
+    for (int t = 0; t < R; t++) {
+      const int r = bitrev<R>(t);
+      dst[(long long)(kb + t * LPS) * N1 + g] = make_float2((float)(vr[r] * scale), (float)(vi[r] * scale));
+    }
   }
 }
 
@@ -562,8 +668,6 @@ inline hipError_t run(const float2* in, float2* out, float2* work, const Seqs& q
       case 4: hipLaunchKernelGGL(stage_kernel<4>, grid, block, 0, st, in, out, work, q, d, J, N, sign, sc); break;
       case 8: hipLaunchKernelGGL(stage_kernel<8>, grid, block, 0, st, in, out, work, q, d, J, N, sign, sc); break;
       case 16: hipLaunchKernelGGL(stage_kernel<16>, grid, block, 0, st, in, out, work, q, d, J, N, sign, sc); break;
-      case 32: hipLaunchKernelGGL(stage_kernel<32>, grid, block, 0, st, in, out, work, q, d, J, N, sign, sc); break;
-      case 64: hipLaunchKernelGGL(stage_kernel<64>, grid, block, 0, st, in, out, work, q, d, J, N, sign, sc); break;
       default: return hipErrorInvalidValue;
     }
     const hipError_t err = hipGetLastError();
