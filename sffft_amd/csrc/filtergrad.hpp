@@ -25,7 +25,7 @@
 // replaced). Bound by VALU issue, about 600 fp32 instructions per lane and transform, and by
 // what hides latency beside it, 2 to 3 wavefronts per SIMD. Measured, that composition before and this
 // kernel now: B=8 H=768 L=1024 fp32 220 -> 20 us (2.5 TB/s of u and dy, 0.5 of a copy), B=6
-// H=513 L=4096 bf16 610 -> 51, B=5 H=320 L=8192 fp32 540 -> 99.
+// H=513 L=4096 bf16 610 -> 51, B=5 H=320 L=8192 fp32 540 -> 88.
 #pragma once
 #include "fftconv.hpp"
 
@@ -150,7 +150,8 @@ struct Geom {
   // Wavefronts per SIMD the register allocation must allow. Three (168 VGPRs) hold the working
   // set; held to four the shorter lengths spill and take 1.2 to 1.8 times as long. At
   // L >= 8192 the LDS allows whole workgroups of 8 or 16 wavefronts only, and two of 8 (128
-  // VGPRs, 50 to 70 of them spilled) beat one: 99 against 105 us at B=5, H=320, L=8192 fp32.
+  // VGPRs, 22 to 43 spilled, mostly the sums during a transform) beat one: 90 against 107 us at
+  // B=5, H=320, L=8192 fp32.
   static constexpr int WPE = T >= 512 ? 4 : 3;
   // a team within one wavefront exchanges without a barrier
   static constexpr bool WAVE = T <= 64;
@@ -255,11 +256,12 @@ __device__ __forceinline__ void forward(const TIO* __restrict__ xa, const TIO* _
                                         const C* w, C w2, bool odd, int t) {
   TIO a[16], b[16];
 #pragma unroll
-  for (int j = 0; j < 16; j++) a[j] = xa[t + G::T * j], b[j] = TIO(0);
+  for (int j = 0; j < 16; j++) a[j] = (xa + G::T * j)[(unsigned)t], b[j] = TIO(0);
   if (xb) {
 #pragma unroll
-    for (int j = 0; j < 16; j++) b[j] = xb[t + G::T * j];
+    for (int j = 0; j < 16; j++) b[j] = (xb + G::T * j)[(unsigned)t];
   }
+  __asm__ volatile("" ::: "memory");
 #pragma unroll
   for (int j = 0; j < 16; j++) x[j] = {io_to_f32(a[j]), io_to_f32(b[j])};
   if (odd) {
@@ -281,7 +283,11 @@ __global__ void __launch_bounds__(Geom<L>::NT, Geom<L>::WPE)
   typedef Geom<L> G;
   constexpr int T = G::T;
   __shared__ C lds[G::TEAMS * G::SLOTS];
-  const int team = threadIdx.x / T, t = threadIdx.x % T;
+  // a team of whole wavefronts is uniform across them: its row pointers are scalars, and a lane adds
+  // one offset for all of its points (an address pair per few points took up to 50 VGPRs, spilled at
+  // L = 2048 and 16384: 48 -> 39 us at B=8, H=768, L=2048 fp32, 200 -> 163 at B=4, H=300, L=16384)
+  const int team = T >= 64 ? __builtin_amdgcn_readfirstlane(threadIdx.x / T) : (int)threadIdx.x / T;
+  const int t = threadIdx.x % T;
   const int half = G::HALVES == 2 ? team & 1 : blockIdx.y;
   const int sub = G::HALVES == 2 ? (team >> 1) % G::SUB : 0;
   const int ch = G::HALVES == 2 ? (team >> 1) / G::SUB : 0;
@@ -369,12 +375,12 @@ __global__ void __launch_bounds__(Geom<L>::NT, Geom<L>::WPE)
       const float* o = reinterpret_cast<const float*>(lds + (team + 1) * G::SLOTS);
       float* d = out + ((size_t)blockIdx.z * H + h) * L;
 #pragma unroll
-      for (int j = 0; j < 16; j++) d[t + T * j] = y[j] + o[t + T * j];
+      for (int j = 0; j < 16; j++) (d + T * j)[(unsigned)t] = y[j] + o[t + T * j];
     }
   } else {
     float* d = out + ((size_t)(blockIdx.z * 2 + half) * H + h) * L;
 #pragma unroll
-    for (int j = 0; j < 16; j++) d[t + T * j] = y[j];
+    for (int j = 0; j < 16; j++) (d + T * j)[(unsigned)t] = y[j];
   }
 }
 
