@@ -346,7 +346,7 @@ def conv(u, kf, plan: Plan, out=None, work=None):
 
 
 def conv_long(u, kf, plan: Plan, out=None, work=None):
-    """Multi-pass convolution (sffft_conv_long_*): three launches on the current stream."""
+    """Multi-pass convolution (sffft_conv_long_*): two or three launches per chunk on the current stream."""
     import torch
 
     u = u.contiguous()

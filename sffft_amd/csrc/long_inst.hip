@@ -46,15 +46,27 @@ static hipError_t launch_long(const void* u, const void* kf, void* y, void* work
   for (int h0 = 0; h0 < H; h0 += chunk) {
     const int nch = H - h0 < chunk ? H - h0 : chunk, pi0 = h0 * BP;
     const unsigned cgrid = (unsigned)((size_t)BP * nch * (NR / LC_CBLOCK));
-    hipLaunchKernelGGL((long_cols_fwd<NC, TIO, CIRC>), dim3(cgrid), dim3(64 * LC_WAVES), 0, s,
-                       static_cast<const TIO*>(u), static_cast<uint32_t*>(work), B, H, NR, pi0, inv_n,
-                       static_cast<const h8*>(ftab));
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
-    const int nrows = nch * NC * BP;
-    hipLaunchKernelGGL((long_rows<R0, R1>), dim3(rows_grid<R0, R1>(nrows)), dim3(64 * LC_WAVES), 0, s,
-                       static_cast<uint32_t*>(work), static_cast<const float4*>(kf), nrows, BP, NC, h0, inv_n,
-                       inv_sqrt_radix<NC>(), static_cast<const h8*>(ftab), static_cast<const float4*>(tw));
+    hipError_t err = hipSuccess;
+    bool fused = false;
+    if constexpr (long_fused<R0, R1, TIO, CIRC>()) {
+      const long long blocks = (long long)BP * nch * (NC / 16);
+      fused = blocks >= LF_MIN_BLOCKS && blocks <= 0x7fffffff;
+      if (fused)
+        hipLaunchKernelGGL((long_cols_rows<NC, R0, R1>), dim3((unsigned)blocks), dim3(64 * LF_WAVES), 0, s,
+                           static_cast<const uint16_t*>(u), static_cast<uint32_t*>(work),
+                           static_cast<const float4*>(kf), B, H, h0, nch, inv_n, static_cast<const h8*>(ftab),
+                           static_cast<const float4*>(tw));
+    }
+    if (!fused) {
+      hipLaunchKernelGGL((long_cols_fwd<NC, TIO, CIRC>), dim3(cgrid), dim3(64 * LC_WAVES), 0, s,
+                         static_cast<const TIO*>(u), static_cast<uint32_t*>(work), B, H, NR, pi0, inv_n,
+                         static_cast<const h8*>(ftab));
+      if ((err = hipGetLastError()) != hipSuccess) return err;
+      const int nrows = nch * NC * BP;
+      hipLaunchKernelGGL((long_rows<R0, R1>), dim3(rows_grid<R0, R1>(nrows)), dim3(64 * LC_WAVES), 0, s,
+                         static_cast<uint32_t*>(work), static_cast<const float4*>(kf), nrows, BP, NC, h0, inv_n,
+                         inv_sqrt_radix<NC>(), static_cast<const h8*>(ftab), static_cast<const float4*>(tw));
+    }
     if ((err = hipGetLastError()) != hipSuccess) return err;
     hipLaunchKernelGGL((long_cols_inv<NC, TIO, CIRC>), dim3(cgrid), dim3(64 * LC_WAVES), 0, s,
                        static_cast<const uint32_t*>(work), static_cast<TIO*>(y), B, H, NR, pi0,

@@ -29,7 +29,7 @@
 //
 // Intermediate: T and U share one workspace, [pair][k1][n2] complex fp16 (4 bytes per
 // point, 4N bytes per pair); U overwrites T row by row. The batch runs in chunks of whole
-// channels (three launches per chunk) sized by the caller's workspace: a workspace that
+// channels (three launches per chunk, or two: long_cols_rows) sized by the caller's workspace: a workspace that
 // fits the Infinity Cache keeps T and U out of HBM. Every value that enters an MFMA
 // is fp16 anyway, so storing fp16 adds no rounding: with fp32 I/O the input enters
 // pass A as an fp16 value plus its fp16 remainder, and there are as many fp16
@@ -38,6 +38,9 @@
 // Circular convolution of period N (CIRC): y[n] = sum_{m<N} x[m] k[(n - m) mod N], rows of
 // length N. The same passes, with pass A contracting over all NC rows and pass C storing
 // all of them; the spectrum is the DFT of the unpadded length-N filter.
+//
+// bf16 chunks of enough workgroups run passes A and B in one launch (long_cols_rows below): T
+// stays in LDS and registers.
 //
 // HBM traffic per pair: pass A reads the two input rows and writes T (4N), pass B reads
 // and rewrites it (8N) and its channel's spectrum (8N per channel, shared by the B/2
@@ -58,7 +61,9 @@ constexpr int LC_CBLOCK = LC_COLS * LC_WAVES;  // columns per column-pass workgr
 
 // w[v] = sc * exp(-2 pi i (e0 + step*v) / N), v = 0..3, N a power of two known at run
 // time (inv_n = 1/N, exact): the base from v_sin/v_cos of the angle reduced to
-// (-1/2, 1/2] revolutions, the others by a complex recurrence (as twiddle4e).
+// (-1/2, 1/2] revolutions, the others by a complex recurrence (as twiddle4e). The fused
+// multiply-adds are written out, here and in cmul_points, so that the fused and the separate
+// passes round alike (which product the compiler contracts is its choice otherwise).
 __device__ __forceinline__ void twiddle4_rt(int e0, int step, int N, float inv_n, float sc, float* wr, float* wi) {
   e0 &= N - 1;
   step &= N - 1;
@@ -70,7 +75,7 @@ __device__ __forceinline__ void twiddle4_rt(int e0, int step, int N, float inv_n
   wi[0] = i;
 #pragma unroll
   for (int v = 1; v < 4; v++) {
-    const float nr = r * sr - i * si, ni = r * si + i * sr;
+    const float nr = __builtin_fmaf(r, sr, -(i * si)), ni = __builtin_fmaf(r, si, i * sr);
     r = nr;
     i = ni;
     wr[v] = r;
@@ -91,8 +96,8 @@ __device__ __forceinline__ u32x4 cmul_points(f4 dr, f4 di, const float* wr, cons
   h8 o;
 #pragma unroll
   for (int v = 0; v < 4; v++) {
-    o[2 * v] = (_Float16)(dr[v] * wr[v] - di[v] * wi[v]);
-    o[2 * v + 1] = (_Float16)(dr[v] * wi[v] + di[v] * wr[v]);
+    o[2 * v] = (_Float16)__builtin_fmaf(dr[v], wr[v], -(di[v] * wi[v]));
+    o[2 * v + 1] = (_Float16)__builtin_fmaf(dr[v], wi[v], di[v] * wr[v]);
   }
   return __builtin_bit_cast(u32x4, o);
 }
@@ -227,27 +232,25 @@ struct LongRowPlan {
   static_assert(LDS_BYTES <= 163840, "tables fit the LDS");
 };
 
+// A row in registers: lane (r, g) of tile (mt, ks) holds n2 = (16ks + 4g + j)*M + 16mt + r.
 template <int R0, int R1>
-__device__ __forceinline__ void long_row(uint32_t* x, const float4* __restrict__ SP, int k1, int N, float inv_n,
-                                         float sc, const h8* F0, const h8* F1, const float4* TW1,
+struct RawRow {
+  uint32_t raw[R1 / 16][R0 / 16][4];
+};
+
+template <int R0, int R1>
+__device__ __forceinline__ void long_row(const RawRow<R0, R1>& row, uint32_t* x, const float4* __restrict__ SP, int k1,
+                                         int N, float inv_n, float sc, const h8* F0, const h8* F1, const float4* TW1,
                                          const float4* TW2, int lane) {
   typedef WavePlan<R0, R1> P;
   constexpr int M = P::M, MT = P::MT, ST = P::ST, KF = R0 / 16;
+  const auto& raw = row.raw;
   constexpr bool TWS = false;  // paired twiddle layout (tw_index): the split one measured 0.5-0.8% slower here
   const int r = lane & 15, g = lane >> 4;
   // compiler-only barrier at the top of each tile step: keeps the next step's table and
   // spectrum reads from being hoisted over the current one (all of them at once would
   // not fit beside the row)
   auto step_fence = [] { __asm__ volatile("" ::: "memory"); };
-
-  // the whole row: lane (r, g) of tile (mt, ks) holds n2 = (16ks + 4g + j)*M + 16mt + r
-  uint32_t raw[MT][KF][4];
-#pragma unroll
-  for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-    for (int ks = 0; ks < KF; ks++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) raw[mt][ks][j] = x[(16 * ks + 4 * g + j) * M + 16 * mt + r];
 
   // ---- phase 1: DFT over n0 (all R0 rows), twiddle -> B2[m tile][k0 strip]. One m tile
   // at a time, so its input dies before the next tile's results are made.
@@ -383,8 +386,165 @@ __global__ void __launch_bounds__(64 * LC_WAVES)
     const int c = ck / NC, k1 = ck - c * NC;
     uint32_t* x = work + ((size_t)(c * BP + bp) * NC + k1) * NR;
     const size_t hk = (size_t)(h0 + c) * NC + k1;  // the spectrum row
-    long_row<R0, R1>(x, kf + hk * (NR / 2), k1, N, inv_n, sc, F0, F1, TW1, TW2, lane);
+    RawRow<R0, R1> in;
+#pragma unroll
+    for (int mt = 0; mt < P::MT; mt++)
+#pragma unroll
+      for (int ks = 0; ks < R0 / 16; ks++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          in.raw[mt][ks][j] = x[(16 * ks + 4 * (lane >> 4) + j) * P::M + 16 * mt + (lane & 15)];
+    long_row<R0, R1>(in, x, kf + hk * (NR / 2), k1, N, inv_n, sc, F0, F1, TW1, TW2, lane);
   }
+}
+
+// ---- passes A and B in one launch ---------------------------------------------------
+// A workgroup of 16 wavefronts takes 16 rows k1 of one pair: it makes them with pass A's column DFTs
+// (all of the pair's input, 16 of the NC results) and each wavefront then runs pass B on one row, held
+// in its registers. T never goes to memory: the columns cross from the lanes that made them to
+// the wavefronts that own their rows through LDS, 16 M columns at a time (one K step of the row's
+// first stage), in two buffers, so that one barrier per step is enough.
+// The NC/16 workgroups of a pair read the same input and the B/2 pairs of a channel the same spectrum rows;
+// they are neighbours on one XCD and take them from its L2. Arithmetic as in the separate
+// passes, in the same order: the results are the same bits. One workgroup per CU (116 KB of LDS, 124 VGPRs
+// at 64x32): bound by the chain of a wavefront's loads, products and LDS exchanges, 31 us a round of 256.
+// B=2 H=768 L=65536 bf16, a chunk of 192 pairs: passes A and B 38 + 81 -> 93 us, the convolution
+// 568 -> 490; L=32768 267 -> 239, B=8 H=300 L=65536 855 -> 695.
+constexpr int LF_WAVES = 16;
+
+// Taken for 2-byte samples, causal filters and row plans whose pass B fits the 128 VGPRs that 16 wavefronts
+// leave each (M = 32: two column tiles a wavefront and step). fp32 samples are twice the bytes to read
+// NC/16 times over, and their value + remainder products spill: B=2 H=768 L=65536 fp32 716 us
+// against 623 in separate passes, L=32768 306 against 306; circular filters contract over twice the rows.
+template <int R0, int R1, class TIO, bool CIRC>
+constexpr bool long_fused() {
+  return sizeof(TIO) == 2 && !CIRC && R1 == 32;
+}
+// ... and for launches of at least 128 workgroups, half the CUs: one workgroup takes some 20 us however few
+// they are, where the separate passes spread their columns and rows over all CUs. L=65536 bf16,
+// separate -> fused: B=2 H=16 (64 workgroups) 28.1 -> 28.8 us, H=32 (128) 33.6 -> 31.1, H=64 51.6 -> 39.7;
+// L=32768 H=32 (128) 25.5 -> 19.8.
+constexpr int LF_MIN_BLOCKS = 128;
+
+// Workgroup -> (channel slot c of the chunk, pair bp, group of 16 rows): a channel's workgroups
+// consecutive on one XCD when the chunk's channels divide among the 8.
+__device__ __forceinline__ void fused_block(int i, int nch, int per, int& c, int& rest) {
+  if ((nch & 7) == 0) {
+    const int x = i & 7, j = i >> 3, q = j / per;
+    c = 8 * q + x;
+    rest = j - q * per;
+  } else {
+    c = i / per;
+    rest = i - c * per;
+  }
+}
+
+template <int NC, int R0, int R1>
+__global__ void __launch_bounds__(64 * LF_WAVES)
+    long_cols_rows(const uint16_t* __restrict__ u, uint32_t* __restrict__ work, const float4* __restrict__ kf, int B, int H,
+                   int h0, int nch, float inv_n, const h8* __restrict__ ftab, const float4* __restrict__ twtab) {
+  typedef WavePlan<R0, R1> P;
+  typedef LongRowPlan<R0, R1> Q;
+  constexpr int M = P::M, MT = P::MT, NR = Q::NR, N = NC * NR, LEN = N / 2;
+  constexpr int NZ = NC / 2, KS = NZ >= 16 ? NZ / 16 : 1;  // non-zero rows n1, K steps over them
+  constexpr int GROUPS = NC / 16, PITCH = 16 * M + 4;        // 4 dwords: the 16 rows on different banks
+  __shared__ float4 lds[Q::TAB_F4];
+  __shared__ __attribute__((aligned(16))) uint32_t slice[2][16 * PITCH];
+  h8* F0 = reinterpret_cast<h8*>(lds);
+  h8* F1 = R1 == R0 ? F0 : F0 + Q::F0_H8;
+  float4* TW1 = lds + Q::F0_H8 + Q::F1_H8;
+  float4* TW2 = P::TW_TABLES == 2 ? TW1 + P::TW_F4 : TW1;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int BP = B >> 1;
+  int c, rest;
+  fused_block(blockIdx.x, nch, BP * GROUPS, c, rest);
+  const int bp = rest / GROUPS, kt = rest - bp * GROUPS, h = h0 + c;
+  const uint16_t* xa = u + ((size_t)(2 * bp) * H + h) * LEN;
+  const uint16_t* xb = xa + (size_t)H * LEN;
+
+  auto tab = [&](int R, int k) { return reinterpret_cast<const float4*>(ftab + cf_off(R) + ((k >> 6) << 7) + (k & 63)); };
+  dma_to_lds<P::TW_TABLES * P::TW_F4, LF_WAVES>(TW1, [&](int k) { return twtab + k; }, lane, wave);
+  dma_to_lds<Q::F0_H8, LF_WAVES>(reinterpret_cast<float4*>(F0), [&](int k) { return tab(R0, k); }, lane, wave);
+  if constexpr (R1 != R0)
+    dma_to_lds<Q::F1_H8, LF_WAVES>(reinterpret_cast<float4*>(F1), [&](int k) { return tab(R1, k); }, lane, wave);
+
+  // Pass A, K step s of row step ks: the lane's two adjacent columns n2 = 16 M ks + 32 wave + 2 r + p
+  // (tile p), rows 16 s + 4 g + j of both sequences, in one 4-byte load each. The next
+  // K step's loads are issued before a step's products.
+  static_assert(MT == 2, "two tiles per wavefront and step");
+  typedef uint16_t pair2 __attribute__((ext_vector_type(2)));
+  pair2 in[8];
+  auto load = [&](int ks, int s) {
+    const int off = 16 * M * ks + 32 * wave + 2 * r;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const int n1 = 16 * s + 4 * g + (j & 3);
+      // rows past NZ (NC = 16) are read again and replaced by zeros below
+      in[j] = *reinterpret_cast<const pair2*>((j < 4 ? xa : xb) + (NZ >= 16 ? n1 : n1 & (NZ - 1)) * NR + off);
+    }
+  };
+  // DFT fragments, held: read per step, they would wait for the loads ahead of them
+  h8 f[KS][2];
+#pragma unroll
+  for (int s = 0; s < KS; s++)
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      f[s][k] = cf_frag<NC, true>(ftab, kt, s, k, lane);
+      __asm__ volatile("" : "+v"(f[s][k]));
+    }
+  load(0, 0);
+  RawRow<R0, R1> row;
+#pragma unroll
+  for (int ks = 0; ks < R0 / 16; ks++) {
+    uint32_t* S = slice[ks & 1];
+    f4 dr[2], di[2];
+    dr[0] = dr[1] = di[0] = di[1] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+      h8 ah[2];
+#pragma unroll
+      for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+          ah[p][j] = (_Float16)(NZ >= 16 || 4 * g + (j & 3) < NZ ? io_to_f32((uint16_t)in[j][p]) : 0.f);
+      __asm__ volatile("" ::: "memory");
+      if (s + 1 < KS)
+        load(ks, s + 1);
+      else if (ks + 1 < R0 / 16)
+        load(ks + 1, 0);
+      __asm__ volatile("" ::: "memory");
+#pragma unroll
+      for (int p = 0; p < 2; p++) {
+        dr[p] = mfma(ah[p], f[s][0], dr[p]);
+        di[p] = mfma(ah[p], f[s][1], di[p]);
+      }
+    }
+    // value v of tile p is column 2 v + p of the lane's eight
+    const int k1 = 16 * kt + r, col = 32 * wave + 8 * g;
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      const int n2 = 16 * M * ks + col + 4 * q;
+      const f4 zr = {dr[0][2 * q], dr[1][2 * q], dr[0][2 * q + 1], dr[1][2 * q + 1]};
+      const f4 zi = {di[0][2 * q], di[1][2 * q], di[0][2 * q + 1], di[1][2 * q + 1]};
+      float wr[4], wi[4];
+      twiddle4_rt(k1 * n2, k1, N, inv_n, inv_sqrt_radix<NC>(), wr, wi);
+      *reinterpret_cast<u32x4*>(S + r * PITCH + col + 4 * q) = cmul_points(zr, zi, wr, wi);
+    }
+    if (ks == R0 / 16 - 1) wait_vmcnt<0>();  // the tables' copies
+    __asm__ volatile("" ::: "memory");
+    __syncthreads();
+    // this wavefront's row, k1 = 16 kt + wave
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) row.raw[mt][ks][j] = S[wave * PITCH + (4 * g + j) * M + 16 * mt + r];
+    __asm__ volatile("" ::: "memory");
+  }
+  const int k1 = 16 * kt + wave;
+  uint32_t* x = work + ((size_t)(c * BP + bp) * NC + k1) * NR;
+  const size_t hk = (size_t)h * NC + k1;  // the spectrum row
+  long_row<R0, R1>(row, x, kf + hk * (NR / 2), k1, N, inv_n, inv_sqrt_radix<NC>(), F0, F1, TW1, TW2, lane);
 }
 
 // ---- pass C: DFT over k1 (all NC rows of U), outputs n1 < NC/2 (all with CIRC) --------

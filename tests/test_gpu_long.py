@@ -222,3 +222,22 @@ def test_complex_input_conv(dev, L, plan_of):
     err = np.linalg.norm(y - ref) / np.linalg.norm(ref)
     print(f"case complex L={L} {plan!r} rel_l2={err:.3e}", flush=True)
     assert err <= 5e-4, (L, repr(plan), err)
+
+
+@pytest.mark.parametrize("L,spec,B,H", [(8192, "16x32x32", 16, 17), (16384, "32x32x32", 6, 24), (32768, "64x32x32", 2, 37),
+                                        (16384, "16x64x32", 2, 136), (65536, "64x64x32", 4, 16)])
+def test_fused_columns_and_rows(dev, L, spec, B, H):
+    """bf16 launches of 128 and more workgroups run the column and row passes in one kernel, smaller ones
+    in two: the same products and roundings in the same order, so the same bits. A one-channel workspace
+    (every chunk below 128 workgroups) takes the separate passes."""
+    import torch
+
+    plan = sf.long_plan(spec)
+    nc = int(spec.split("x")[0])
+    assert H * (B // 2) * (nc // 16) >= 128 > (B // 2) * (nc // 16)
+    u, k = oracle.gen_inputs(B, H, L, seed=31)
+    one = torch.empty((B // 2) * 2 * L * 4, dtype=torch.uint8, device=dev)
+    whole = torch.empty(H * one.numel(), dtype=torch.uint8, device=dev)
+    a = _run(dev, u, k, plan, "bf16", work=one)
+    b = _run(dev, u, k, plan, "bf16", work=whole)
+    assert np.array_equal(a, b)
