@@ -24,7 +24,7 @@
 // moved 8 bytes a sample 11 times each way. Two wavefronts per SIMD (the fp64 planes take the
 // LDS) leave it bound by the latency between the barriers of the stages, so every launch requests
 // its points before it evaluates its tables. Measured at B=8, H=16, 256 x 256: 269 us in 13
-// launches -> 72 us.
+// launches -> 65 us.
 #pragma once
 #include "transforms.hpp"
 

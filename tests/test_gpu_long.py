@@ -14,6 +14,8 @@ the same bound, and the bench configurations run at full B=8, H=768 through the
 bit-exact properties of test_gpu_configs.py (permutation of pairs and channels,
 repeatability) on sampled sequences.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -238,6 +240,16 @@ def test_fused_columns_and_rows(dev, L, spec, B, H):
     u, k = oracle.gen_inputs(B, H, L, seed=31)
     one = torch.empty((B // 2) * 2 * L * 4, dtype=torch.uint8, device=dev)
     whole = torch.empty(H * one.numel(), dtype=torch.uint8, device=dev)
-    a = _run(dev, u, k, plan, "bf16", work=one)
-    b = _run(dev, u, k, plan, "bf16", work=whole)
-    assert np.array_equal(a, b)
+    x = sf.to_bf16(torch.from_numpy(u).to(dev))
+    kf = sf.spectrum(torch.from_numpy(k).to(dev), L, plan)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for entry in (sf.lib().sffft_conv_long_bf16, sf.lib().sffft_corr_long_bf16):
+        out = []
+        for work in (one, whole):
+            y = torch.empty_like(x)
+            assert entry(ptr(x), ptr(kf), ptr(y), ptr(work), work.numel(), B, H, L, ctypes.byref(plan), stream) == sf.SFFFT_OK
+            out.append(y)
+        assert torch.equal(out[0], out[1])
+    ref = oracle.conv(u[:2, :1], k[:1])
+    assert oracle.rel_l2(sf.conv(x, kf, plan, work=whole)[:2, :1].float().cpu().numpy(), ref) <= BOUND["bf16"]
