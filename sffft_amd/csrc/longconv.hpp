@@ -63,7 +63,9 @@ constexpr int LC_CBLOCK = LC_COLS * LC_WAVES;  // columns per column-pass workgr
 // time (inv_n = 1/N, exact): the base from v_sin/v_cos of the angle reduced to
 // (-1/2, 1/2] revolutions, the others by a complex recurrence (as twiddle4e). The fused
 // multiply-adds are written out, here and in cmul_points, so that the fused and the separate
-// passes round alike (which product the compiler contracts is its choice otherwise).
+// passes round alike (which product the compiler contracts is its choice otherwise): here the
+// products with the imaginary part are the fused ones, in cmul_points the first of each sum.
+// Other choices flip fp16 roundings of the outputs, 5e-4 of a bf16 result.
 __device__ __forceinline__ void twiddle4_rt(int e0, int step, int N, float inv_n, float sc, float* wr, float* wi) {
   e0 &= N - 1;
   step &= N - 1;
@@ -75,7 +77,7 @@ __device__ __forceinline__ void twiddle4_rt(int e0, int step, int N, float inv_n
   wi[0] = i;
 #pragma unroll
   for (int v = 1; v < 4; v++) {
-    const float nr = __builtin_fmaf(r, sr, -(i * si)), ni = __builtin_fmaf(r, si, i * sr);
+    const float nr = __builtin_fmaf(-i, si, r * sr), ni = __builtin_fmaf(i, sr, r * si);
     r = nr;
     i = ni;
     wr[v] = r;
