@@ -229,6 +229,25 @@ __device__ __forceinline__ void twiddle4e(int e0, int step, float sc, float* wr,
     wi[v] = i;
   }
 }
+// w[v] = exp(-2*pi*i * (e0 + STEP*v) / N): the step's factor is a constant (v_sin/v_cos of it would be
+// less exact). Negative inv_n: the conjugates.
+template <int N, int STEP>
+__device__ __forceinline__ void twiddle4c(int e0, float* wr, float* wi, float inv_n) {
+  static_assert(STEP > 0 && STEP < N / 2, "a positive sine");
+  e0 &= N - 1;
+  const float x0 = (float)(e0 > N / 2 ? e0 - N : e0) * inv_n;
+  const float c = cos_rev(STEP * (1.0f / N)), s = __builtin_copysignf(sin_rev(STEP * (1.0f / N)), inv_n);
+  const float s0 = sin_rev(x0);
+  wr[0] = cos_rev(x0);
+  wi[0] = -s0;
+  wr[1] = __builtin_fmaf(wr[0], c, -(s * s0));
+  wi[1] = __builtin_fmaf(s0, -c, -(s * wr[0]));
+#pragma unroll
+  for (int v = 2; v < 4; v++) {
+    wr[v] = __builtin_fmaf(s, wi[v - 1], c * wr[v - 1]);
+    wi[v] = __builtin_fmaf(wi[v - 1], c, -(s * wr[v - 1]));
+  }
+}
 // (r, i) *= (fr, fi), four values
 __device__ __forceinline__ void cmul4(float* r, float* i, const float* fr, const float* fi) {
 #pragma unroll
@@ -781,7 +800,7 @@ __device__ __forceinline__ void phase2_s3(_Float16* re, _Float16* im, const floa
   if constexpr (REC) {
     const int m0 = 4 * g * R2 + c;  // lane value v: m = m0 + v R2
     twiddle4e<N>(wave * ROWS * m0, wave * ROWS * R2, sc1, lr, li, inv_n);
-    twiddle4e<N>(m0, R2, 1.f, fr, fi, inv_n);
+    twiddle4c<N, R2>(m0, fr, fi, inv_n);
   }
   // Two forms of the same row loop. One row per step keeps the loop that the multi-tile
   // plans were tuned with: the several-row form, even with one row per step, changes how

@@ -90,3 +90,26 @@ def test_one_sequence_results_do_not_depend_on_the_wavefronts(dev, L, spec, io):
         u = sf.to_bf16(u)
     y = [sf.conv(u, sf.spectrum(k, L, p), p) for p in (sf.make_plan(spec, 4), sf.make_plan(spec, 8))]
     assert torch.equal(*y)
+
+
+# sha256 (first 16 digits) of the outputs, fp32 and bf16, of seeded inputs at the plans that step their last
+# twiddles from row to row: the factor of a step is a constant, which v_sin/v_cos at run time would
+# only approximate (1e-5 of the outputs).
+PINNED_BITS = [(4096, "32x16x16", 4, 2, "4eab10d83cb29ff1", "3296fb094d284c25"),
+               (8192, "64x16x16", 8, 2, "8777a28b67dea942", "315159c27c50da98"),
+               (8192, "64x16x16", 8, 1, "973c9be0dd82ce2f", "59c9e5401573f798")]
+
+
+@pytest.mark.parametrize("L,spec,waves,seqs,fp32,bf16", PINNED_BITS)
+def test_output_bits(dev, L, spec, waves, seqs, fp32, bf16):
+    import hashlib
+
+    import torch
+
+    plan = sf.make_plan(spec, waves, seqs=seqs)
+    u, k = oracle.gen_inputs(4, 5, L, seed=L + waves)
+    kf = sf.spectrum(torch.from_numpy(k).to(dev), L, plan)
+    x = torch.from_numpy(u).to(dev)
+    for xi, pin in ((x, fp32), (sf.to_bf16(x), bf16)):
+        y = sf.conv(xi, kf, plan)
+        assert hashlib.sha256(y.view(torch.uint8).cpu().numpy().tobytes()).hexdigest()[:16] == pin, xi.dtype
