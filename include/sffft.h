@@ -35,6 +35,8 @@ extern "C" {
  * {16,32,64}. Mirrors Plan<R0,R1,R2> and the W template argument of fftconv
  * (src/sffft.cu:92-104, 243-245, 507-513).
  *   waves : wavefronts (64 lanes) per workgroup
+ *           (32x16x16, seqs = 1, waves = 8, cached = 1: 4 where a call has several workgroups
+ *           per CU, which is then faster; the results are the same bits)
  *   acc   : 0 = fp32 accumulation, 1 = fp16 accumulation ("fp16acc" methods)
  *   cached: 1 = DFT matrices from the coefficient table ("kernel_cached"),
  *           0 = computed in the kernel ("kernel_legacy")  (src/sffft.cu:253-265)

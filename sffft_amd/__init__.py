@@ -198,11 +198,11 @@ DEFAULT_PLANS = {
 }
 # Multi-pass plans (mode 2): column radix x row plan, measured at B=8, H=768
 LONG_DEFAULT_PLANS = {32768: "64x32x32", 65536: "64x64x32", 131072: "64x64x64"}
-# One sequence per transform (workgroup kernel) for an odd batch. The results do not depend on the
-# wavefronts; measured (us, fp32 / bf16): 4096 (B=3, H=859) 4 wavefronts 55.0 / 42.9, 8 62.5 / 46.6;
-# 8192 (B=5, H=320) 8 wavefronts 67.5 / 59.0, 4 70.0 / 62.2.
+# One sequence per transform (workgroup kernel) for an odd batch. 8192: 8 wavefronts, whose results are
+# those of 4, took 0.90 to 1.00 of the time of 4 over B = 1..15, H = 64..1536 in both I/O types
+# (B=5, H=320 fp32 62.3 -> 60.2 us, B=7, H=768 bf16 185 -> 179). 4096: see filled_waves in conv_inst.hip.
 ODD_BATCH_PLANS = {128: ("16x16", 2), 256: ("32x16", 2), 512: ("32x32", 2), 1024: ("64x32", 4),
-                   2048: ("16x16x16", 8), 4096: ("32x16x16", 4), 8192: ("32x32x16", 8), 16384: ("32x32x32", 8)}
+                   2048: ("16x16x16", 8), 4096: ("32x16x16", 8), 8192: ("32x32x16", 8), 16384: ("32x32x32", 8)}
 
 
 def long_plan(spec: str) -> Plan:

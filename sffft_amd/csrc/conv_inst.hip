@@ -21,20 +21,45 @@ constexpr int fused_wpe() {
   return CACHED && P::R0 == 64 && P::R1 == 16 && P::R2 == 16 && NW == 8 ? lds_waves_per_simd<P, NW>() : 1;
 }
 
-template <class P, int NW, int NSEQ, class TIO, bool CACHED>
-static hipError_t launch_fused(const void* u, const void* kf, void* y, int B, int H, const void* ftab, const void*,
-                               int acc16, int corr, hipStream_t stream) {
+// Wavefronts a plan's workgroups run with once a call fills the CUs; 0: its own. One-sequence 32x16x16
+// with 8 wavefronts has the same results, bit for bit, with 4 that evaluate every row's twiddles (EACH), and
+// the smaller workgroups are faster as soon as several share a CU: 8 -> 4 wavefronts, fp32 / bf16, 768
+// workgroups 19.6 -> 18.0 / 15.1 -> 14.2 us, 2577 (B=3, H=859) 62.5 -> 55.0 / 46.6 -> 42.9, 6000 (B=15) 112.5 ->
+// 100.2 / 81.2 -> 78.7; 264 11.6 -> 11.8 / 10.8 -> 9.7; but 192 7.5 -> 8.2 / 6.6 -> 7.1. So from more than one
+// workgroup per CU on, with fp32 I/O (whose two workgroups of 8 still run at a time) from more than two.
+template <class P, int NW, int NSEQ, bool CACHED>
+constexpr int filled_waves() {
+  return CACHED && NSEQ == 1 && P::R0 == 32 && P::R1 == 16 && P::R2 == 16 && NW == 8 ? 4 : 0;
+}
+
+template <class P, int NW, int NSEQ, class TIO, bool CACHED, int WPE, bool EACH>
+static void launch_fused_waves(const void* u, const void* kf, void* y, int B, int H, const void* ftab, int acc16,
+                               int corr, hipStream_t stream) {
   const unsigned grid = (unsigned)(H * (B / NSEQ));
-  constexpr int WPE = fused_wpe<P, NW, CACHED>();
   const float inv_n = (corr ? -1.f : 1.f) / (float)P::N;  // exact: N is a power of two
   if (acc16)
-    hipLaunchKernelGGL((fftconv_kernel<P, NW, NSEQ, TIO, CACHED, true, WPE>), dim3(grid), dim3(64 * NW), 0, stream,
+    hipLaunchKernelGGL((fftconv_kernel<P, NW, NSEQ, TIO, CACHED, true, WPE, EACH>), dim3(grid), dim3(64 * NW), 0, stream,
                        static_cast<const TIO*>(u), static_cast<const float2*>(kf), static_cast<TIO*>(y), B, H,
                        static_cast<const h8*>(ftab), inv_n);
   else
-    hipLaunchKernelGGL((fftconv_kernel<P, NW, NSEQ, TIO, CACHED, false, WPE>), dim3(grid), dim3(64 * NW), 0, stream,
+    hipLaunchKernelGGL((fftconv_kernel<P, NW, NSEQ, TIO, CACHED, false, WPE, EACH>), dim3(grid), dim3(64 * NW), 0, stream,
                        static_cast<const TIO*>(u), static_cast<const float2*>(kf), static_cast<TIO*>(y), B, H,
                        static_cast<const h8*>(ftab), inv_n);
+}
+
+template <class P, int NW, int NSEQ, class TIO, bool CACHED>
+static hipError_t launch_fused(const void* u, const void* kf, void* y, int B, int H, const void* ftab, const void*,
+                               int acc16, int corr, hipStream_t stream) {
+  constexpr int FILLED = filled_waves<P, NW, NSEQ, CACHED>(), CUS = 256;
+  if constexpr (FILLED > 0) {
+    if ((long long)H * (B / NSEQ) > CUS * (int)(sizeof(TIO) / 2)) {
+      launch_fused_waves<P, FILLED, NSEQ, TIO, CACHED, fused_wpe<P, FILLED, CACHED>(), true>(u, kf, y, B, H, ftab, acc16,
+                                                                                             corr, stream);
+      return hipGetLastError();
+    }
+  }
+  launch_fused_waves<P, NW, NSEQ, TIO, CACHED, fused_wpe<P, NW, CACHED>(), false>(u, kf, y, B, H, ftab, acc16, corr,
+                                                                                 stream);
   return hipGetLastError();
 }
 

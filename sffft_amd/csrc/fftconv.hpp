@@ -686,7 +686,7 @@ __device__ __forceinline__ void pack_operand(const float* xr, const float* xi, h
   }
 }
 
-template <class P, int NW, int NSEQ, bool CACHED, int SPLITS>
+template <class P, int NW, bool CACHED, int SPLITS, bool EACH>
 __device__ __forceinline__ void phase2_s3(_Float16* re, _Float16* im, const float2* __restrict__ K,
                                           const h8* __restrict__ ftab, int acc16, float inv_n, int lane, int wave) {
   constexpr int R0 = P::R0, R1 = P::R1, R2 = P::R2, N = P::N, T1 = R1 / 16, T2 = R2 / 16;
@@ -791,11 +791,9 @@ __device__ __forceinline__ void phase2_s3(_Float16* re, _Float16* im, const floa
   // factor w^m: with one tile per axis the wavefront evaluates the first row's and the
   // factors once, and steps from row to row with one complex product per value. It holds
   // 16 more VGPRs through the rows: measured faster with 8 rows per wavefront (64x16x16),
-  // slower with 4 (32x16x16, where it costs a workgroup per CU). 32x16x16 with 4 wavefronts and one
-  // sequence per transform evaluates every row's: 1-2% slower, but then its results are those of
-  // 8 wavefronts bit for bit, which it replaces for odd batches (13% faster: B=3, H=859, L=4096
-  // fp32 62.5 -> 55.0 us, bf16 46.6 -> 42.9), and 0.07% closer to fp64 than by recurrence.
-  constexpr bool REC = T1 * T2 == 1 && ROWS >= 8 && !(NSEQ == 1 && R0 == 32);
+  // slower with 4 (32x16x16, where it costs a workgroup per CU). EACH: every row's are evaluated,
+  // which makes the results those of twice the wavefronts bit for bit.
+  constexpr bool REC = T1 * T2 == 1 && ROWS >= 8 && !EACH;
   float lr[4], li[4], fr[4], fi[4];
   if constexpr (REC) {
     const int m0 = 4 * g * R2 + c;  // lane value v: m = m0 + v R2
@@ -1140,7 +1138,7 @@ constexpr int fp32_splits() {
 // scheduling block per tile. WPE is the wavefronts per SIMD the register allocation
 // must allow (the LDS-limited occupancy, or 1 for no limit): without it the schedule
 // of the longer blocks can take more VGPRs than that occupancy leaves.
-template <class P, int NW, int NSEQ, class TIO, bool CACHED, bool ACC16, int WPE>
+template <class P, int NW, int NSEQ, class TIO, bool CACHED, bool ACC16, int WPE, bool EACH = false>
 __global__ void __launch_bounds__(64 * NW, WPE)
     fftconv_kernel(const TIO* __restrict__ u, const float2* __restrict__ kf, TIO* __restrict__ y, int B, int H,
                    const h8* __restrict__ ftab, float inv_n) {
@@ -1174,7 +1172,8 @@ __global__ void __launch_bounds__(64 * NW, WPE)
   } else {
     phase1<P, NW, NSEQ, TIO, CACHED, SPLIT_IN>(ad, fr, re, im, ftab, acc16, inv_n, lane, wave);
     __syncthreads();
-    phase2_s3<P, NW, NSEQ, CACHED, sizeof(TIO) == 4 && !ACC16 ? fp32_splits<P>() : 0>(re, im, K, ftab, acc16, inv_n, lane, wave);
+    phase2_s3<P, NW, CACHED, sizeof(TIO) == 4 && !ACC16 ? fp32_splits<P>() : 0, EACH>(re, im, K, ftab, acc16, inv_n,
+                                                                                     lane, wave);
   }
   __syncthreads();
   phase3<P, NW, NSEQ, TIO, CACHED>(y + row_a, y + row_b, re, im, ftab, acc16, lane, wave);

@@ -78,18 +78,30 @@ def test_legacy_and_fp16_accumulation(dev, L):
                     assert np.isfinite(err) and err <= bound(io, acc, p.seqs), (L, repr(p), io, err)
 
 
+@pytest.mark.parametrize("acc", [0, 1])
 @pytest.mark.parametrize("io", ["fp32", "bf16"])
 @pytest.mark.parametrize("L,spec", [(4096, "32x16x16"), (8192, "32x32x16")])
-def test_one_sequence_results_do_not_depend_on_the_wavefronts(dev, L, spec, io):
-    """The odd-batch plans' wavefront count is a matter of speed only: bit-identical results."""
+def test_one_sequence_results_do_not_depend_on_the_wavefronts(dev, L, spec, io, acc):
+    """The odd-batch plans' wavefront count is a matter of speed only: bit-identical results. At L = 4096
+    a call of more than 256 (bf16) or 512 (fp32) workgroups runs on 4 wavefronts, a smaller one on 8."""
     import torch
 
-    u, k = oracle.gen_inputs(3, 5, L, seed=L)
-    u, k = torch.from_numpy(u).to(dev), torch.from_numpy(k).to(dev)
+    H = 172 if L == 4096 else 5
+    un, kn = oracle.gen_inputs(3, H, L, seed=L)
+    u, k = torch.from_numpy(un).to(dev), torch.from_numpy(kn).to(dev)
     if io == "bf16":
         u = sf.to_bf16(u)
-    y = [sf.conv(u, sf.spectrum(k, L, p), p) for p in (sf.make_plan(spec, 4), sf.make_plan(spec, 8))]
-    assert torch.equal(*y)
+    p = sf.make_plan(spec, 8, acc=acc)
+    y = sf.conv(u, sf.spectrum(k, L, p), p)
+    if L == 4096:
+        assert repr(p) == repr(sf.default_plan(L, io, 3, acc=acc))
+        few = [sf.conv(u[:, h : h + 43].contiguous(), sf.spectrum(k[h : h + 43], L, p), p) for h in range(0, H, 43)]
+        other = torch.cat(few, 1)
+    else:
+        p = sf.make_plan(spec, 4, acc=acc)
+        other = sf.conv(u, sf.spectrum(k, L, p), p)
+    assert torch.equal(y, other)
+    assert oracle.rel_l2(y[:, :3].float().cpu().numpy(), oracle.conv(un[:, :3], kn[:3])) <= bound(io, acc)
 
 
 # sha256 (first 16 digits) of the outputs, fp32 and bf16, of seeded inputs at the plans that step their last
@@ -97,7 +109,8 @@ def test_one_sequence_results_do_not_depend_on_the_wavefronts(dev, L, spec, io):
 # only approximate (1e-5 of the outputs).
 PINNED_BITS = [(4096, "32x16x16", 4, 2, "4eab10d83cb29ff1", "3296fb094d284c25"),
                (8192, "64x16x16", 8, 2, "8777a28b67dea942", "315159c27c50da98"),
-               (8192, "64x16x16", 8, 1, "973c9be0dd82ce2f", "59c9e5401573f798")]
+               (8192, "64x16x16", 8, 1, "973c9be0dd82ce2f", "59c9e5401573f798"),
+               (4096, "32x16x16", 4, 1, "2842d07a9863d8a6", "bbae65dc377ec5d0")]
 
 
 @pytest.mark.parametrize("L,spec,waves,seqs,fp32,bf16", PINNED_BITS)
