@@ -124,7 +124,7 @@ int sffft_corr_long_bf16(const uint16_t* u, const void* kf, uint16_t* y, void* w
  * for L a power of two in [128, 16384] and any B, H. No counterpart in the reference: it serves
  * the gradient of sffft_conv_* with respect to k. u, dy are [B][H][L] (fp32 or bf16, rows of any
  * element alignment), dk is [H][L] fp32, 16-byte aligned, and may overlap neither input. The
- * transforms and sums are fp32 (about 2e-7 rel-L2 against fp64). `work` (16-byte aligned,
+ * transforms and sums are fp32 (3e-7 to 7e-7 rel-L2 against fp64, whatever the rows' relative sizes). `work` (16-byte aligned,
  * clobbered) must hold sffft_filter_grad_work_bytes(B, H, L) bytes and may be NULL if that is 0.
  * Needs no plan and no table: the first call may be captured. */
 size_t sffft_filter_grad_work_bytes(int B, int H, int L);

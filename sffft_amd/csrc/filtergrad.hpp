@@ -6,7 +6,10 @@
 // whatever its batch: with U_b and D_b the zero-padded 2L-point spectra of the rows,
 // dk = IDFT(sum_b D_b conj(U_b)). Two batch rows travel as one complex row, z = x_b + i x_b+1:
 // then Re IDFT(Z_dy conj(Z_u)) is already the sum of both rows' correlations (the cross terms
-// are the imaginary part), so the pair is never taken apart.
+// are the imaginary part), so the pair is never taken apart. The cross terms still round: dy of one row
+// times u of the other may be far larger than either row's own product. So where they differ, row b + 1
+// of u is scaled by a power of two to the size of row b, and that row of dy by its inverse
+// (balance()): the sum is unchanged, and each cross term is bounded by a row's own product.
 //
 // The 2L-point transform of a row whose second half is zero splits into two L-point ones,
 // its even bins (the transform of x) and its odd bins (of x[n] w_2L^n), and
@@ -20,13 +23,16 @@
 // order, so nothing is ever permuted, and the lane that ends with a bin of u also ends with that bin
 // of dy: spectra, products and their sum stay in registers.
 //
-// fp32 throughout: 3e-7 to 6e-7 from 64 bits, where fp16 operands gave 2e-4 to 3.4e-4 (the
-// composition of the spectrum of every row, a convolution and a sum over b, which this
+// fp32 throughout: 3e-7 (L = 128) to 7e-7 (L = 16384) from 64 bits, also for rows 1e12 apart in size (1e-5
+// at a ratio of 100 and 0.2 at 1e6 without the balance, which costs 0 to 4% of the time), where fp16
+// operands gave 2e-4 to 3.4e-4 (the composition of the spectrum of every row, a convolution and a sum over b, which this
 // replaced). Bound by VALU issue, about 600 fp32 instructions per lane and transform, and by
 // what hides latency beside it, 2 to 3 wavefronts per SIMD. Measured, that composition before and this
 // kernel now: B=8 H=768 L=1024 fp32 220 -> 20 us (2.5 TB/s of u and dy, 0.5 of a copy), B=6
-// H=513 L=4096 bf16 610 -> 51, B=5 H=320 L=8192 fp32 540 -> 88.
+// H=513 L=4096 bf16 610 -> 53, B=5 H=320 L=8192 fp32 540 -> 88.
 #pragma once
+#include <type_traits>
+
 #include "fftconv.hpp"
 
 namespace sffft {
@@ -186,17 +192,15 @@ __device__ __forceinline__ C root(int num, int den) {  // exp(-2 pi i num / den)
   return {c, -s};
 }
 
-// Radix-16 stages on REST-point blocks, REST > 16: butterfly, twiddle, exchange; then the last
-// stage of radix REST <= 16. On entry x holds the lane's 16 points of this stage.
+// Radix-16 stages on REST-point blocks, REST > 16, after the first (forward()): butterfly, twiddle,
+// exchange; then the last stage of radix REST <= 16.
 template <class G, int REST, int S>
 __device__ __forceinline__ void forward_stage(C* x, C* buf, const C* w, int t) {
   if constexpr (REST > 16) {
     constexpr int sJ = REST / 16;
     C* at = buf + slot_base<sJ>(t);
-    if constexpr (S > 0) {
 #pragma unroll
-      for (int j = 0; j < 16; j++) x[j] = at[slot_off<sJ>(j)];
-    }
+    for (int j = 0; j < 16; j++) x[j] = at[slot_off<sJ>(j)];
     fft<16, false>(x);
     twiddle16<false, true>(x, w[S]);
 #pragma unroll
@@ -248,29 +252,146 @@ __device__ __forceinline__ void inverse_stage(C* x, C* buf, const C* w, int t) {
   }
 }
 
+// Sum of v over groups of W consecutive lanes (2 to 64): in each of their lanes, for W = 64 as a scalar.
+template <int W>
+__device__ __forceinline__ float lane_sum(float v) {
+  auto dpp = [](float x, auto ctrl, auto rows) {
+    constexpr int c = decltype(ctrl)::value, m = decltype(rows)::value;
+    const int b = __builtin_bit_cast(int, x);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, b, c, m, 0xf, false));
+  };
+  constexpr std::integral_constant<int, 0xf> all{};
+  v += dpp(v, std::integral_constant<int, 0xb1>{}, all);                            // lane ^ 1
+  if constexpr (W >= 4) v += dpp(v, std::integral_constant<int, 0x4e>{}, all);    // lane ^ 2
+  if constexpr (W >= 8) v += dpp(v, std::integral_constant<int, 0x141>{}, all);   // mirrored in 8: the other four
+  if constexpr (W >= 16) v += dpp(v, std::integral_constant<int, 0x140>{}, all);  // in 16: the other eight
+  if constexpr (W == 32) v += __shfl_xor(v, 16);
+  if constexpr (W == 64) {  // lane 15 to the next 16 lanes, lane 31 to the next 32
+    v += dpp(v, std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});
+    v += dpp(v, std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+    v = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+  }
+  return v;
+}
+
+// The balance of a pair: the power of two that takes the size of its second row (the imaginary
+// parts) towards that of the first, as its exponent. A row's size is the root of the sum of its
+// lanes' largest squares (within a factor of 4 of its norm). Pairs whose rows are within a factor of 8 of
+// each other in every lane, as equal rows are, keep their scale: what they cost is lane_sizes() and a
+// vote. Others are taken to within a factor of 2, by at most 2^48: beside a row of zeros too, whose dy would
+// only round; fp32 keeps the inverse factor in range for dy up to 1e24.
+__device__ __forceinline__ float2 lane_sizes(const C* x) {
+  float a = 0.f, b = 0.f;
+#pragma unroll
+  for (int j = 0; j < 16; j += 2) {
+    a = fmaxf(fmaxf(fabsf(x[j].r), fabsf(x[j + 1].r)), a);
+    b = fmaxf(fmaxf(fabsf(x[j].i), fabsf(x[j + 1].i)), b);
+  }
+  return make_float2(a, b);
+}
+__device__ __forceinline__ bool unequal(float2 s) {  // by about a factor of 8 (bit patterns 3 exponents apart)
+  const unsigned d = __builtin_bit_cast(unsigned, s.x) - __builtin_bit_cast(unsigned, s.y);
+  return d + (3u << 23) > 6u << 23;
+}
+template <class G>
+__device__ __forceinline__ int balance(float2 size2) {
+  int ea = __builtin_bit_cast(int, size2.x) >> 23, eb = __builtin_bit_cast(int, size2.y) >> 23;  // not negative
+  if constexpr (G::T >= 64) {
+    ea = __builtin_amdgcn_readfirstlane(ea);
+    eb = __builtin_amdgcn_readfirstlane(eb);
+  }
+  const int k = (ea - eb) / 2;
+  return k < -48 ? -48 : k > 48 ? 48 : k;
+}
+__device__ __forceinline__ float pow2(int k) { return __builtin_bit_cast(float, (127 + k) << 23); }
+
+// A team of several wavefronts: its wavefronts' sizes, and the latest pair with unequal rows.
+template <int T>
+struct Sizes {
+  float2 wave[T > 64 ? T / 64 : 1];
+  int vote;
+};
+
 // Forward transform of one half of the pair of rows xa, xb (xb null: a zero row). The odd half
 // is the transform of z[n] w_2L^n at n = t + T j: w_2L^(T j) = w_32^j is a constant, and the
 // lane's common factor w_2L^t goes through the first butterfly, to its outputs (w2).
-template <class G, class TIO>
+// U: of u, which sets the pair's balance k; otherwise of dy. Teams of several wavefronts vote across
+// the first stage's barrier, and the rare pair that is to be scaled runs that stage again: a barrier
+// before it would keep the wavefronts whose rows have arrived from starting (5% at L = 16384).
+template <class G, bool U, class TIO>
 __device__ __forceinline__ void forward(const TIO* __restrict__ xa, const TIO* __restrict__ xb, C* x, C* buf,
-                                        const C* w, C w2, bool odd, int t) {
-  TIO a[16], b[16];
+                                        Sizes<G::T>* sizes, int pair, const C* w, C w2, bool odd, int t, int& k) {
+  auto load = [&](int t) {
+    TIO a[16], b[16];
 #pragma unroll
-  for (int j = 0; j < 16; j++) a[j] = (xa + G::T * j)[(unsigned)t], b[j] = TIO(0);
-  if (xb) {
+    for (int j = 0; j < 16; j++) a[j] = (xa + G::T * j)[(unsigned)t], b[j] = TIO(0);
+    if (xb) {
 #pragma unroll
-    for (int j = 0; j < 16; j++) b[j] = (xb + G::T * j)[(unsigned)t];
+      for (int j = 0; j < 16; j++) b[j] = (xb + G::T * j)[(unsigned)t];
+    }
+    __asm__ volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < 16; j++) x[j] = {io_to_f32(a[j]), io_to_f32(b[j])};
+  };
+  auto scale = [&](int e) {
+    const float c = pow2(e);
+#pragma unroll
+    for (int j = 0; j < 16; j++) x[j].i *= c;
+  };
+  auto first_stage = [&](int t) {
+    if (odd) {
+#pragma unroll
+      for (int j = 1; j < 16; j++) x[j] = rot32<false>(x[j], j);
+#pragma unroll
+      for (int j = 0; j < 16; j++) x[j] = mul(x[j], w2);
+    }
+    C* at = buf + slot_base<G::T>(t);
+    fft<16, false>(x);
+    twiddle16<false, true>(x, w[0]);
+#pragma unroll
+    for (int v = 0; v < 16; v++) at[slot_off<G::T>(v)] = x[slot<16>(v)];
+    team_sync<G>();
+  };
+  constexpr int W = G::T < 64 ? G::T : 64;
+  load(t);
+  if constexpr (U) {
+    k = 0;
+    if (xb) {
+      float2 s = lane_sizes(x);
+      const uint64_t v = __ballot(unequal(s));
+      if (v) {
+        if constexpr (G::T > 64) {
+          sizes->vote = pair;
+        } else {
+          s = make_float2(lane_sum<W>(s.x * s.x), lane_sum<W>(s.y * s.y));
+          const uint64_t mine = W == 64 ? v : v >> (threadIdx.x & 63 & ~(W - 1)) & ((1ull << (W & 63)) - 1);
+          k = mine ? balance<G>(s) : 0;
+        }
+      }
+    }
   }
-  __asm__ volatile("" ::: "memory");
-#pragma unroll
-  for (int j = 0; j < 16; j++) x[j] = {io_to_f32(a[j]), io_to_f32(b[j])};
-  if (odd) {
-#pragma unroll
-    for (int j = 1; j < 16; j++) x[j] = rot32<false>(x[j], j);
-#pragma unroll
-    for (int j = 0; j < 16; j++) x[j] = mul(x[j], w2);
+  if (k) scale(U ? k : -k);
+  first_stage(t);
+  if constexpr (U && G::T > 64) {
+    if (xb && __builtin_amdgcn_readfirstlane(sizes->vote) == pair) {
+      // on a lane index of its own, so that nothing of this block is made ahead of it and kept: at T = 1024,
+      // where registers are shortest, all of it, below only the slots (the rest is shared with the first
+      // time: 157 against 166 us at B=4, H=300, L=16384 fp32, but 92 against 88 at B=5, H=320, L=8192)
+      int l = t;
+      __asm__ volatile("" : "+v"(l));
+      const int lane = G::T > 512 ? l : t;
+      load(lane);
+      float2 s = lane_sizes(x);
+      s = make_float2(lane_sum<W>(s.x * s.x), lane_sum<W>(s.y * s.y));
+      if ((l & 63) == 0) sizes->wave[l >> 6] = s;
+      team_sync<G>();
+      s = sizes->wave[l & (G::T / 64 - 1)];
+      k = balance<G>(make_float2(lane_sum<G::T / 64>(s.x), lane_sum<G::T / 64>(s.y)));
+      scale(k);
+      first_stage(lane);
+    }
   }
-  forward_stage<G, G::L, 0>(x, buf, w, t);
+  forward_stage<G, G::L / 16, 1>(x, buf, w, t);
 }
 
 // grid: (channel groups, halves from the grid, batch splits). Partial results (one per half
@@ -283,6 +404,7 @@ __global__ void __launch_bounds__(Geom<L>::NT, Geom<L>::WPE)
   typedef Geom<L> G;
   constexpr int T = G::T;
   __shared__ C lds[G::TEAMS * G::SLOTS];
+  __shared__ fg::Sizes<T> sizes_[T > 64 ? G::TEAMS : 1];
   // a team of whole wavefronts is uniform across them: its row pointers are scalars, and a lane adds
   // one offset for all of its points (an address pair per few points took up to 50 VGPRs, spilled at
   // L = 2048 and 16384: 48 -> 39 us at B=8, H=768, L=2048 fp32, 200 -> 163 at B=4, H=300, L=16384)
@@ -294,6 +416,11 @@ __global__ void __launch_bounds__(Geom<L>::NT, Geom<L>::WPE)
   const int h = blockIdx.x * G::CH + ch;
   const bool live = h < H;
   C* buf = lds + team * G::SLOTS;
+  fg::Sizes<T>* sizes = sizes_ + (T > 64 ? team : 0);
+  if constexpr (T > 64) {
+    if (t == 0) sizes->vote = -1;
+    __syncthreads();
+  }
   const int pairs = (B + 1) / 2, p0 = blockIdx.z * pairs_per_split;
   const int np = pairs - p0 < pairs_per_split ? pairs - p0 : pairs_per_split;
 
@@ -321,8 +448,9 @@ __global__ void __launch_bounds__(Geom<L>::NT, Geom<L>::WPE)
     const size_t row = ((size_t)b * H + (live ? h : H - 1)) * L;
     const size_t next = b + 1 < B ? (size_t)H * L : 0;
     C xu[16], xd[16];
-    forward<G, TIO>(u + row, next ? u + row + next : nullptr, xu, buf, w, w2, half != 0, t);
-    forward<G, TIO>(dy + row, next ? dy + row + next : nullptr, xd, buf, w, w2, half != 0, t);
+    int k;
+    forward<G, true>(u + row, next ? u + row + next : nullptr, xu, buf, sizes, r, w, w2, half != 0, t, k);
+    forward<G, false>(dy + row, next ? dy + row + next : nullptr, xd, buf, sizes, r, w, w2, half != 0, t, k);
     if (mine) {
 #pragma unroll
       for (int v = 0; v < 16; v++) {

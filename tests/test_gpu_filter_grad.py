@@ -63,6 +63,52 @@ def test_matches_fp64(dev, L, io):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("L", sf.LENGTHS)
+def test_rows_of_unequal_size(dev, L):
+    """Two batch rows share a transform: the error of a row must not depend on its partner's size. Rows of
+    u scaled by s and 1/s in turn and those of dy by the inverse leave every row's product as it is, so the
+    bound is that of equal rows; rows of few samples and empty ones beside dense ones likewise."""
+    g = torch.Generator(device=dev).manual_seed(L + 1)
+
+    def check(u, dy, what):
+        ref = reference(u, dy)
+        err = ((torch.ops.sffft.filter_grad(u, dy).double().cpu() - ref).norm(dim=1) / ref.norm(dim=1)).max().item()
+        assert err <= 2e-6, (what, err)  # as in test_matches_fp64
+
+    for B, H in ((2, 3), (5, 4), (16, 3)):
+        for s in (3.0, 30.0, 1000.0, 1e6):
+            u, dy = (torch.randn(B, H, L, device=dev, generator=g) for _ in range(2))
+            c = torch.tensor([s if b % 2 else 1 / s for b in range(B)], device=dev)[:, None, None]
+            check(u * c, dy / c, (B, H, s))
+            check(u / c, dy * c, (B, H, 1 / s))
+    u, dy = (torch.randn(4, 3, L, device=dev, generator=g) for _ in range(2))
+    u[0::2] = 0
+    u[0::2, :, 5] = 1.0
+    dy[1::2] /= 100 * L**0.5
+    check(u, dy, "single samples")
+    u[2] = 0
+    u[1] = 0
+    check(u, dy, "empty rows")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L", [128, 256, 512, 1024, 2048, 16384])
+def test_channels_are_independent(dev, L):
+    """Unequal, infinite or NaN rows of one channel leave the other channels' bits alone, though channels
+    share workgroups and, below L = 1024, wavefronts."""
+    g = torch.Generator(device=dev).manual_seed(L + 2)
+    u, dy = (torch.randn(5, 6, L, device=dev, generator=g) for _ in range(2))
+    base = torch.ops.sffft.filter_grad(u, dy)
+    for bad in (1e4, float("inf"), float("nan")):
+        v = u.clone()
+        v[1, 2] *= bad
+        out = torch.ops.sffft.filter_grad(v, dy)
+        keep = [h for h in range(6) if h != 2]
+        assert torch.equal(out[keep], base[keep]), bad
+        assert torch.isfinite(out[2]).all().item() == (bad == 1e4)
+
+
+@pytest.mark.gpu
 def test_any_alignment_and_stride(dev):
     """Rows at any element offset, and non-contiguous operands, as the composed path took them."""
     x = torch.randn(4 * 3 * 512 + 1, device=dev)
