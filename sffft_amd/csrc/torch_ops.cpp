@@ -123,7 +123,17 @@ at::Tensor corr_gpu(const at::Tensor& u, const at::Tensor& kf, c10::IntArrayRef 
   return run_conv(u, kf, plan, true);
 }
 
-at::Tensor longconv_gpu(const at::Tensor& u, const at::Tensor&, const at::Tensor& kf, c10::IntArrayRef plan) {
+at::Tensor longconv_gpu(const at::Tensor& u, const at::Tensor& k, const at::Tensor& kf, c10::IntArrayRef plan) {
+  // what the backward pass needs, refused here rather than there: the filter's gradient has k's shape and
+  // type, and a kernel for these lengths only
+  TORCH_CHECK(u.dim() == 3 && k.dim() == 2 && k.size(0) == u.size(1) && k.size(1) == u.size(2) &&
+                  k.scalar_type() == at::kFloat && k.device() == u.device(),
+              "sffft::longconv: k must be the [H, L] float32 filter of u [B, H, L] on its device, got ", k.sizes(), " ",
+              k.scalar_type(), " for u of shape ", u.sizes());
+  const int64_t L = u.size(2);
+  TORCH_CHECK(L >= 128 && L <= 16384 && (L & (L - 1)) == 0,
+              "sffft::longconv: L must be a power of two from 128 to 16384, got ", L,
+              " (LongConv takes the multi-pass lengths)");
   return run_conv(u, kf, plan, false);
 }
 

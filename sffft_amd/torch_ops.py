@@ -73,6 +73,10 @@ def _corr_fake(u, kf, plan):
 
 @torch.library.register_fake("sffft::longconv")
 def _longconv_fake(u, k, kf, plan):
+    torch._check(u.dim() == 3 and k.dim() == 2 and k.shape[0] == u.shape[1] and k.shape[1] == u.shape[2],
+                 lambda: "k must be the [H, L] filter of u")
+    torch._check(k.dtype == torch.float32, lambda: "k must be float32")
+    torch._check(u.shape[2] in LENGTHS, lambda: "L must be a power of two from 128 to 16384")
     return _conv_fake(u, kf, plan)
 
 

@@ -41,6 +41,41 @@ def test_fake_shapes():
         assert y.shape == (8, 768, 1024) and y.dtype == torch.bfloat16
 
 
+def _refused_longconv_calls(device):
+    """(u, k, kf, plan) that sffft::longconv must refuse when it is called, not in its backward pass."""
+    def t(*shape, dtype=torch.float32):
+        return torch.empty(*shape, device=device, dtype=dtype)
+
+    p, long = (torch_ops.plan_fields(sf.default_plan(L, "fp32", 2)) for L in (256, 32768))
+    kf = t(3, 512, dtype=torch.complex64)
+    return [(t(2, 3, 256), t(4, 256), kf, p),                        # k of other channels
+            (t(2, 3, 256), t(3, 128), kf, p),                        # of another length
+            (t(2, 3, 256), t(1, 3, 256), kf, p),
+            (t(2, 3, 256), t(3, 256, dtype=torch.float64), kf, p),
+            (t(2, 3, 256), t(3, 256, dtype=torch.bfloat16), kf, p),
+            (t(2, 1, 32768), t(1, 32768), t(1, 65536, dtype=torch.complex64), long)]  # a multi-pass length
+
+
+def test_longconv_refuses_while_tracing():
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    with FakeTensorMode():
+        for args in _refused_longconv_calls("cuda"):
+            with pytest.raises(RuntimeError):
+                torch.ops.sffft.longconv(*args)
+
+
+@pytest.mark.gpu
+def test_longconv_refuses_at_the_call(dev):
+    for u, k, kf, plan in _refused_longconv_calls(dev):
+        with pytest.raises(RuntimeError):
+            torch.ops.sffft.longconv(u, k.requires_grad_(), kf, plan)
+    u, k = torch.zeros(2, 3, 256, device=dev), torch.zeros(3, 256)
+    p = torch_ops.plan_fields(sf.default_plan(256, "fp32", 2))
+    with pytest.raises(RuntimeError):  # the filter on another device
+        torch.ops.sffft.longconv(u, k, torch.ops.sffft.spectrum(k.to(dev), p), p)
+
+
 @pytest.mark.parametrize("L", sf.LENGTHS + sf.LONG_LENGTHS)
 def test_default_plans_are_compiled(L):
     for io in ("fp32", "bf16"):
