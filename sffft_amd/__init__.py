@@ -588,7 +588,7 @@ class RocfftPipeline:
 # (mode 2, long_inst.hip, which also include the single-pass headers).
 SINGLE_PASS_SOURCES = ("csrc/fftconv.hpp", "csrc/fftconv_wave.hpp", "csrc/registry.hpp", "csrc/plans.def",
                        "csrc/conv_inst.hip", "Makefile")
-MULTI_PASS_SOURCES = SINGLE_PASS_SOURCES + ("csrc/longconv.hpp", "csrc/long_inst.hip")
+MULTI_PASS_SOURCES = SINGLE_PASS_SOURCES + ("csrc/longconv.hpp", "csrc/longmap.hpp", "csrc/long_inst.hip")
 
 
 def _code_only(rel: str, text: str) -> str:

@@ -50,7 +50,7 @@ static hipError_t launch_long(const void* u, const void* kf, void* y, void* work
     bool fused = false;
     if constexpr (long_fused<R0, R1, TIO, CIRC>()) {
       const long long blocks = (long long)BP * nch * (NC / 16);
-      fused = blocks >= LF_MIN_BLOCKS && blocks <= 0x7fffffff;
+      fused = fused_launch(blocks, NC, R0);
       if (fused)
         hipLaunchKernelGGL((long_cols_rows<NC, R0, R1>), dim3((unsigned)blocks), dim3(64 * LF_WAVES), 0, s,
                            static_cast<const uint16_t*>(u), static_cast<uint32_t*>(work),

@@ -47,6 +47,7 @@
 // pairs through L2), pass C reads U (4N) and writes the two output rows.
 #pragma once
 #include "fftconv_wave.hpp"
+#include "longmap.hpp"
 
 // k0 strips per phase-2 step of the row pass (pass B)
 #ifndef LONG_ROW_STRIPS
@@ -407,7 +408,7 @@ __global__ void __launch_bounds__(64 * LC_WAVES)
 // the wavefronts that own their rows through LDS, 16 M columns at a time (one K step of the row's
 // first stage), in two buffers, so that one barrier per step is enough.
 // The NC/16 workgroups of a pair read the same input and the B/2 pairs of a channel the same spectrum rows;
-// they are neighbours on one XCD and take them from its L2. Arithmetic as in the separate
+// as neighbours on one XCD (fused_block) they take them from its L2. Arithmetic as in the separate
 // passes, in the same order: the results are the same bits. One workgroup per CU (116 KB of LDS, 124 VGPRs
 // at 64x32): bound by the chain of a wavefront's loads, products and LDS exchanges, 31 us a round of 256.
 // B=2 H=768 L=65536 bf16, a chunk of 192 pairs: passes A and B 38 + 81 -> 93 us, the convolution
@@ -422,24 +423,7 @@ template <int R0, int R1, class TIO, bool CIRC>
 constexpr bool long_fused() {
   return sizeof(TIO) == 2 && !CIRC && R1 == 32;
 }
-// ... and for launches of at least 128 workgroups, half the CUs: one workgroup takes some 20 us however few
-// they are, where the separate passes spread their columns and rows over all CUs. L=65536 bf16,
-// separate -> fused: B=2 H=16 (64 workgroups) 28.1 -> 28.8 us, H=32 (128) 33.6 -> 31.1, H=64 51.6 -> 39.7;
-// L=32768 H=32 (128) 25.5 -> 19.8.
-constexpr int LF_MIN_BLOCKS = 128;
-
-// Workgroup -> (channel slot c of the chunk, pair bp, group of 16 rows): a channel's workgroups
-// consecutive on one XCD when the chunk's channels divide among the 8.
-__device__ __forceinline__ void fused_block(int i, int nch, int per, int& c, int& rest) {
-  if ((nch & 7) == 0) {
-    const int x = i & 7, j = i >> 3, q = j / per;
-    c = 8 * q + x;
-    rest = j - q * per;
-  } else {
-    c = i / per;
-    rest = i - c * per;
-  }
-}
+// (Which launches: fused_launch.)
 
 template <int NC, int R0, int R1>
 __global__ void __launch_bounds__(64 * LF_WAVES)
@@ -459,9 +443,8 @@ __global__ void __launch_bounds__(64 * LF_WAVES)
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int BP = B >> 1;
-  int c, rest;
-  fused_block(blockIdx.x, nch, BP * GROUPS, c, rest);
-  const int bp = rest / GROUPS, kt = rest - bp * GROUPS, h = h0 + c;
+  const FusedBlock at = fused_block<GROUPS>(blockIdx.x, nch, BP, fused_grouped(gridDim.x, nch));
+  const int c = at.c, bp = at.bp, kt = at.kt, h = h0 + c;
   const uint16_t* xa = u + ((size_t)(2 * bp) * H + h) * LEN;
   const uint16_t* xb = xa + (size_t)H * LEN;
 

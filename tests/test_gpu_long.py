@@ -227,7 +227,10 @@ def test_complex_input_conv(dev, L, plan_of):
 
 
 @pytest.mark.parametrize("L,spec,B,H", [(8192, "16x32x32", 16, 17), (16384, "32x32x32", 6, 24), (32768, "64x32x32", 2, 37),
-                                        (16384, "16x64x32", 2, 136), (65536, "64x64x32", 4, 16)])
+                                        (16384, "16x64x32", 2, 136), (65536, "64x64x32", 4, 16),
+                                        # more workgroups than CUs, channels no multiple of 8
+                                        (8192, "16x32x32", 30, 21), (16384, "32x32x32", 10, 31), (32768, "64x32x32", 14, 11),
+                                        (65536, "64x64x32", 12, 13)])
 def test_fused_columns_and_rows(dev, L, spec, B, H):
     """bf16 launches of 128 and more workgroups run the column and row passes in one kernel, smaller ones
     in two: the same products and roundings in the same order, so the same bits. A one-channel workspace
