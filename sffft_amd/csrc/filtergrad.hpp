@@ -156,7 +156,7 @@ struct Geom {
   // Wavefronts per SIMD the register allocation must allow. Three (168 VGPRs) hold the working
   // set; held to four the shorter lengths spill and take 1.2 to 1.8 times as long. At
   // L >= 8192 the LDS allows whole workgroups of 8 or 16 wavefronts only, and two of 8 (128
-  // VGPRs, 22 to 43 spilled, mostly the sums during a transform) beat one: 90 against 107 us at
+  // VGPRs, 27 to 47 spilled, mostly the sums during a transform) beat one: 90 against 107 us at
   // B=5, H=320, L=8192 fp32.
   static constexpr int WPE = T >= 512 ? 4 : 3;
   // a team within one wavefront exchanges without a barrier

@@ -90,9 +90,10 @@ def filter_grad(u: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
     """dk[h, j] = sum_b sum_{n >= j} dy[b, h, n] u[b, h, n - j] for u, dy [B, H, L] (fp32 [H, L]).
 
     Up to L = 16384 one fused kernel (``torch.ops.sffft.filter_grad``), which sums the batch's
-    spectra before a channel's one inverse transform. It records no gradient, so a dy whose own
-    gradient is being recorded (a second derivative) takes the composition of the differentiable
-    operators below, as the multi-pass lengths (L > 16384) do.
+    spectra before a channel's one inverse transform. That operator records no gradient, so a dy
+    whose own gradient is being recorded takes the composition of the differentiable operators
+    below, as the multi-pass lengths (L > 16384) do. (``torch.ops.sffft.longconv`` has an adjoint
+    of its own for its second derivative and does not come here.)
 
     The composition computes per sequence the convolution of dy with the conjugate spectrum of u
     (the correlation of the two; the conjugation is folded into the spectrum's gather), summed

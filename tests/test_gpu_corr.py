@@ -88,14 +88,16 @@ def test_third_derivative(dev):
     assert ((dc - ref).norm() / ref.norm()).item() <= 1e-6
 
 
-@pytest.mark.gpu
-def test_backward_capture_after_an_eager_forward(dev):
-    """The conjugate tables exist once the forward ones do: a capture of the backward pass needs no
-    eager backward before it. (A wave plan no other test of this process runs with these radices.)"""
-    L = 512
-    plan = sf.make_plan("64x16", 12, seqs=2, mode=1, channels=3)
+BACKWARD_CAPTURE = """
+import torch
+import sffft_amd as sf
+from sffft_amd import torch_ops
+
+L = 512
+for plan in (sf.make_plan("64x16", 12, seqs=2, mode=1, channels=3), sf.default_plan(L), sf.long_plan("32x32x32")):
+    L = plan.r0 * plan.r1 * plan.r2 // 2
     p = torch_ops.plan_fields(plan)
-    u, k = torch.randn(2, 3, L, device=dev), torch.randn(3, L, device=dev)
+    u, k = torch.randn(2, 3, L, device="cuda"), torch.randn(3, L, device="cuda")
     kf = torch.ops.sffft.spectrum(k, p)
     torch.ops.sffft.conv(u, kf, p)
     torch.cuda.synchronize()
@@ -111,3 +113,18 @@ def test_backward_capture_after_an_eager_forward(dev):
         torch.cuda.synchronize()
         assert torch.equal(y, torch.ops.sffft.corr(u, kf, p))
         assert torch.equal(dk, torch.ops.sffft.filter_grad(u, u))
+print("captured")
+"""
+
+
+@pytest.mark.gpu
+def test_backward_capture_after_an_eager_forward(dev):
+    """The conjugate tables exist once the forward ones do: a capture of the backward pass needs no
+    eager backward before it. In a process of its own, which has run no backward pass of any plan."""
+    import os
+    import subprocess
+    import sys
+
+    r = subprocess.run([sys.executable, "-c", BACKWARD_CAPTURE], capture_output=True, text=True, timeout=100,
+                       cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert r.returncode == 0 and "captured" in r.stdout, r.stderr[-2000:]

@@ -141,11 +141,19 @@ def test_race_check_build_agrees(dev, L):
 
 
 @pytest.mark.gpu
-def test_second_derivative_takes_the_composed_path(dev):
-    """With the gradient's own gradient recorded, d(dk)/d(dy) is still there."""
+@pytest.mark.parametrize("composed", [False, True])
+def test_second_derivative(dev, composed):
+    """With the gradient's own gradient recorded, d(dk)/d(dy) is still there: through LongConv's backward
+    pass, whose fused filter gradient has an adjoint of its own, and through torch_ops.filter_grad on a dy
+    that records a gradient, which takes the composition of differentiable operators."""
     u, k = torch.randn(2, 3, 256, device=dev), torch.randn(3, 256, device=dev, requires_grad=True)
     dy = torch.randn(2, 3, 256, device=dev, requires_grad=True)
-    (dk,) = torch.autograd.grad(torch_ops.LongConv()(u, k), k, dy, create_graph=True)
+    if composed:
+        dk = torch_ops.filter_grad(u, dy)
+        ref = reference(u, dy.detach())
+        assert ((dk.detach().double().cpu() - ref).norm() / ref.norm()).item() <= 5e-4  # fp16 operands
+    else:
+        (dk,) = torch.autograd.grad(torch_ops.LongConv()(u, k), k, dy, create_graph=True)
     c = torch.randn(3, 256, device=dev)
     (g,) = torch.autograd.grad((dk * c).sum(), dy)
     # d/d(dy) of sum_j c[h, j] dk[h, j]: the causal convolution of u with c
