@@ -604,7 +604,7 @@ int spectrum_impl(const float* kr, const float* ki, int H, int L, int klen, cons
                      ki ? ki + off : nullptr, w, klen, N, n);
   int st = hip_status(hipGetLastError(), "spectrum pad launch");
   if (st) return st;
-  const xf::Seqs q{H, 1, 0, N, 1, 0};
+  const xf::Seqs q{H, H, N, 0, 1, 0};
   float2* scratch = N <= xf::ONEPASS_MAX_N ? nullptr : static_cast<float2*>(kf) + (size_t)h0 * N;
   if ((st = hip_status(xf::run(w, w, scratch, q, N, 0, 1.f, s), "spectrum transform launch"))) return st;
   return permute_launch(w, static_cast<float2*>(kf), H, plan, whole, conj, s, h0);

@@ -235,6 +235,11 @@ struct LineGeom {
   static constexpr int LDS = SLOTS + SLOTS / 16 + (EXTRA ? 16 : 0);
   // From N = 256 the first stage loads runs of 128 bytes and more straight into registers.
   static constexpr bool DIRECT = N >= 256;
+  // Sequences of 8 and 16 points leave through LDS: a lane's stores of its own sequence, 64 and 128 bytes from
+  // the next lane's, took 36.2 and 38.2 us for 2^23 points and 6.95 and 7.26 for 2^14; runs across the lanes 24.0,
+  // 24.2, 5.14 and 5.11 (part of it the addresses, see line_kernel). Of 2 and 4 points the direct stores, 16 and
+  // 32 bytes apart, take 22.2 and 25.9 for 2^23.
+  static constexpr bool STAGED = N == 8 || N == 16;
   // twiddle bases of the non-last stages: w_N^j for j < N / 16 (w_Nj^inner = w_N^(inner N/Nj))
   static constexpr int TW = N / MAX_RADIX > 1 ? N / MAX_RADIX : 1;
   // radix of the stage whose remaining product of radices is REST (16s first)
@@ -342,6 +347,9 @@ __global__ void __launch_bounds__(LineGeom<N>::THREADS)
   constexpr int R = LG::last(), LPS = N / R;
   const long long s0 = (long long)blockIdx.x * LG::G;
   const int G = q.nseq - s0 < LG::G ? (int)(q.nseq - s0) : LG::G;
+  // run_lines' sequences lie at one distance: Seqs::base's 64-bit divisions, one for each element on the way in, took
+  // 2.2 us of a small call (6.9 -> 4.7 at 4096 x 4) and 2 to 4 of 2^23 points
+  auto base = [&](int g) { return (s0 + g) * q.dist_inner; };
   // the first stage's line of this lane: points inner + sJ t of sequence s0 + gt, in flight while
   // the tables are evaluated
   constexpr int sJ = LG::DIRECT ? N / MAX_RADIX : 1;
@@ -350,7 +358,7 @@ __global__ void __launch_bounds__(LineGeom<N>::THREADS)
   if constexpr (LG::DIRECT) {
     // lanes past the last sequence repeat it and store nothing: a zero instead of the load, chosen
     // per point, became a branch and a wait per point
-    const float2* src = in + q.base(s0 + (gt < G ? gt : G - 1)) + inner;
+    const float2* src = in + base(gt < G ? gt : G - 1) + inner;
 #pragma unroll
     for (int t = 0; t < MAX_RADIX; t++) x[t] = src[t * sJ];
     __asm__ volatile("" ::: "memory");
@@ -379,7 +387,7 @@ __global__ void __launch_bounds__(LineGeom<N>::THREADS)
   } else {
     for (int i = threadIdx.x; i < LG::SLOTS; i += LG::THREADS) {
       const int g = i / N;
-      buf[lpad(i)] = g < G ? in[q.base(s0 + g) + (i - g * N)] : make_float2(0.f, 0.f);
+      buf[lpad(i)] = g < G ? in[base(g) + (i - g * N)] : make_float2(0.f, 0.f);
     }
     __syncthreads();
     line_stages<N, N>(buf, tc, ts, sign);
@@ -395,14 +403,24 @@ __global__ void __launch_bounds__(LineGeom<N>::THREADS)
       vi[t] = (double)v.y;
     }
     line_dft<R>(vr, vi, sign);
-    if (g < G) {
-      float2* dst = out + q.base(s0 + g) + kb;
+    if constexpr (LG::STAGED) {
+#pragma unroll
+      for (int k = 0; k < R; k++) {
+        const int r = bitrev<R>(k);
+        buf[lpad(at + k)] = make_float2((float)(vr[r] * scale), (float)(vi[r] * scale));
+      }
+    } else if (g < G) {
+      float2* dst = out + base(g) + kb;
 #pragma unroll
       for (int k = 0; k < R; k++) {
         const int r = bitrev<R>(k);
         dst[k * LPS] = make_float2((float)(vr[r] * scale), (float)(vi[r] * scale));
       }
     }
+  }
+  if constexpr (LG::STAGED) {
+    lds_sync();
+    for (int i = threadIdx.x; i < G * N; i += LG::THREADS) out[base(i / N) + i % N] = buf[lpad(i)];
   }
 }
 
@@ -413,7 +431,7 @@ inline void launch_line(const float2* in, float2* out, const Seqs& q, int sign, 
 }
 
 inline bool run_lines(const float2* in, float2* out, const Seqs& q, int N, int sign, float scale, hipStream_t st) {
-  if (q.stride != 1 || q.seq_fast) return false;
+  if (q.stride != 1 || q.seq_fast || q.inner != q.nseq) return false;
   switch (N) {
     case 2: launch_line<2>(in, out, q, sign, scale, st); return true;
     case 4: launch_line<4>(in, out, q, sign, scale, st); return true;
@@ -659,6 +677,7 @@ inline hipError_t run(const float2* in, float2* out, float2* work, const Seqs& q
   const int sign = inverse ? 1 : -1;
   if (N <= ONEPASS_MAX_N && run_lines(in, out, q, N, sign, scale, st)) return hipGetLastError();
   if (run_two_pass(in, out, work, q, N, sign, scale, st)) return hipGetLastError();
+  if (d.S > 1 && !work) return hipErrorInvalidValue;
   for (int J = 0; J < d.S; J++) {
     const long long threads = q.nseq * (N / d.r[J]);
     const dim3 grid((unsigned)((threads + 127) / 128)), block(128);

@@ -76,6 +76,37 @@ def test_one_pass_matches_staged_path_bitwise(batch, N):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (N, inverse)
 
 
+@pytest.mark.parametrize("N", [2, 4, 8, 16, 32, 128, 512])
+@pytest.mark.parametrize("groups,more", [(0, 1), (1, -1), (1, 0), (2, 3)])
+def test_one_pass_workgroups_and_gaps(groups, more, N):
+    """A workgroup of the one-pass kernel takes 4096 / N sequences: one sequence, the last workgroup not quite full,
+    full, and three sequences into a third one, packed, in place and with a gap between sequences that stays as it
+    was; all bit for bit the staged kernels' results on the same values as columns."""
+    batch = groups * (4096 // N) + more
+    print(f"one-pass batch={batch} N={N}", flush=True)
+    x = crandn(np.random.default_rng(7 * N + batch), batch, N)
+    cols = sf.fft(torch.from_numpy(np.ascontiguousarray(x.T)).to(DEV), dim=0).cpu().numpy()
+    want = np.ascontiguousarray(cols.T).view(np.uint32)
+    rows = torch.from_numpy(x).to(DEV)
+    assert np.array_equal(sf.fft(rows).cpu().numpy().view(np.uint32), want)
+
+    work = torch.empty(batch * N, dtype=torch.complex64, device=DEV)
+
+    def c_fft(src, dst, dist):
+        assert sf.lib().sffft_fft_c2c(src.data_ptr(), dst.data_ptr(), work.data_ptr(), batch * N * 8, batch, N, 1,
+                                      dist, 0, 1.0, torch.cuda.current_stream().cuda_stream) == 0
+        return dst.cpu().numpy()
+
+    dist = N + 3
+    gaps = np.full((batch, dist), 9 - 4j, np.complex64)
+    gaps[:, :N] = x
+    out = c_fft(torch.from_numpy(gaps).to(DEV), torch.full((batch, dist), 5 + 1j, dtype=torch.complex64, device=DEV),
+                dist)
+    assert np.array_equal(np.ascontiguousarray(out[:, :N]).view(np.uint32), want)
+    assert (out[:, N:] == np.complex64(5 + 1j)).all()
+    assert np.array_equal(c_fft(rows, rows, N).view(np.uint32), want)
+
+
 @pytest.mark.parametrize("batch,N", [(2, 1 << 15), (3, 1 << 16), (2, 1 << 17), (2, 1 << 19), (2, 1 << 20),
                                      (2, 1 << 21), (2, 1 << 24)])
 def test_two_pass_matches_staged_path_bitwise(batch, N):
