@@ -334,8 +334,8 @@ __device__ __forceinline__ int line_position(int f) {
 }
 
 // Measured (768 x 16384, 1536 x 8192, 6144 x 2048, 49152 x 256): with the sequence staged through LDS
-// on the way in and out and the roots of unity in LDS 97.5, 93, 83 and 71 us; this 64, 53, 41 and
-// 35 (3.1 to 5.7 TB/s of calls on three inputs in turn; a copy 5.2). At N >= 8192 one or two workgroups fill a CU and the
+// on the way in and out and the roots of unity in LDS 97.5, 93, 83 and 71 us; this 64, 49, 40 and
+// 35 (3.2 to 5.8 TB/s of calls on three inputs in turn; a copy 5.2). At N >= 8192 one or two workgroups fill a CU and the
 // round trips to memory at either end of a sequence show. Workgroups that stay and request the next
 // sequence while they transform one spill (18 to 22 VGPRs at 128) and took 76 and 77 us.
 template <int N>
